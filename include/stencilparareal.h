@@ -56,7 +56,7 @@ extern "C" {
 #define SP_KERNEL_AUTO -1
 #define SP_KERNEL_SCALAR 0 /* one column per lane, any sizes and storage types */
 #define SP_KERNEL_PAIR 1   /* two x-adjacent columns per lane: FP64 (16-byte accesses) or FP32 arithmetic over FP32 / BF16 storage */
-#define SP_KERNEL_QUAD 2   /* FP64, 2x2 columns per lane in stages 1-3 (32x32 tiles, 512 threads) */
+#define SP_KERNEL_QUAD 2   /* FP64, 2x2 columns per lane (32x32 tiles) */
 #define SP_KERNEL_SPLIT 3  /* FP64, two launches of a two-stage x-pair kernel through a work field */
 
 /*
@@ -118,12 +118,11 @@ int sp_prop_set_upwind(sp_prop* p, int upwind);
 /* SP_PATH_FUSED (default) or SP_PATH_STAGED for DoRK4. */
 int sp_prop_set_path(sp_prop* p, int path);
 /* Fused-kernel choice: variant SP_KERNEL_*, tile tx x ty columns, nthreads per block,
- * kchunk planes per block (0: whole k extent; the quad variant runs an odd kchunk as
- * kchunk + 1, with the same results).  variant SP_KERNEL_AUTO restores the
+ * kchunk planes per block (0: whole k extent).  variant SP_KERNEL_AUTO restores the
  * built-in choice.  Compiled shapes: scalar {32x32x1024, 32x24x1024, 24x24x1024,
  * 32x16x512, 16x16x256}, pair {32x32x512, 32x16x512, 16x16x256}, quad {32x32x512}
- * (the built-in choice for FP64 launches of 256 or more blocks; FP32 / BF16 storage takes
- * the pair kernel in its place), split {32x32x512,
+ * (its blocks run 768 threads; the built-in choice for FP64 launches of 256 or more
+ * blocks; FP32 / BF16 storage takes the pair kernel in its place), split {32x32x512,
  * 32x16x512, 32x16x256, 16x16x256}.  The split variant (FP64 fields, even ni) runs each
  * step as two launches through a work field the propagator allocates (8 bytes per point
  * of the batch) when the tile is chosen; its results equal the other FP64 variants' bit

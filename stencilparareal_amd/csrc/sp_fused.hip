@@ -1036,166 +1036,251 @@ __device__ __forceinline__ void rk4_half_pair_body(const HalfArgs& h, const int 
     }
 }
 
-// ---- FP64 2x2 variant (32x32 tiles, 512 threads) -----------------------------------------
-// Stages 1-3 give each lane a 2x2 block of columns (an x pair in two consecutive rows).  The
-// centres of one row are y neighbours of the other, so 10 ds_read_b128 per block and stage
-// give what the pair layout reads with 14; the points per lane (4 + 4 + 4 + 2) and with
-// them the register budget are the pair kernel's.  Stage 4 keeps the pair layout.
-// Bank conflicts: a lane row of VW blocks steps W 16-byte chunks per block row (two plane
-// rows of W/2 chunks), so a plane stride W = VW (mod 16) puts consecutive lanes on
-// consecutive chunks across row ends, for reads (input plane) and writes (output plane)
-// alike.  VW = 22 (stage 1's 22 blocks per row), plane strides 54 and 38 doubles.  In
-// stages 2 and 3 the lanes past a row's last block are spare: they read the input plane's
-// padding columns (so their groups keep the same chunk pattern) and write nothing.
-// q: stage 1 keeps it in registers, stages 2 and 3 load it from global memory at lags 5
-// and 8 (one plane ahead), stage 3 forwards it to stage 4 through the LDS plane Q4.
-// The q plane for P0 is loaded two planes ahead: at one plane (~1.9 us at 16 x 128^3) the
-// loads' HBM latency still showed, 4-9 % of the step.
+// ---- FP64 2x2 variant (32x32 tiles, 12 waves) --------------------------------------------
+// A lane owns one 2x2 block of columns (an x pair in two consecutive rows) in every stage it
+// takes part in, and the four stages are divided between the waves:
+//   waves 0-5, 7   stages 1 and 2      waves 8-11   stages 3 and 4
+//   wave 6         stage 1 on its outermost ring and stage 3 on its ring
+// Regions in blocks: stage 4 is the tile's 16x16 blocks; the star reaches one block (two
+// cells) per stage along one axis only, so stage 3 needs those and the 64 blocks beside them
+// (no corners), stage 2 68 more, stage 1 72 more: 460, 388, 320, 256 blocks.  The order
+//   0-255 the tile, 256-319, 320-383, 384-447 the sides of rings 1-3, 448-459 the diagonals
+//   (four of stage 2 first)
+// gives every wave two stage steps per plane and every SIMD (waves w, w+4, w+8) six, against
+// 7 for square regions with all stages in every wave.
+// A lane's own values pass from stage to stage in registers: the centres of stages 2 and 4,
+// and q at lags 2 and 4 (stages 1, 2; read once from LDS) and 7 and 10 (stages 3, 4; loaded
+// once from global memory into a ring of four).  Of the sums, only the planes that have x and
+// y terms still to come or z terms missing are kept; the first two z terms are taken from the
+// centres when a plane's turn comes.  So 162 registers hold two stages, three waves per SIMD.
+// What a plane costs (counted in the assembly): 120 VALU instructions per wave, all FP64, and
+// per CU 218 ds_read_b128, 40 ds_write_b128 and 37 wave-wide global accesses.  Measured alone
+// those are about 1600 cycles of VALU per SIMD, 1150 + 560 of LDS and 600 of the memory path;
+// a plane takes about 2750, and the clock drops from 2.4 to 2.0-2.15 GHz under it, so the step
+// is bound by VALU, LDS and power together, not by HBM.
+// Reads are issued a part ahead of the arithmetic that uses them, and stage 1's x and y
+// neighbours before the plane's barrier: the q planes sit in four buffers used in turn, so no
+// one writes what those reads still fetch.  The q plane goes from global memory straight into
+// LDS (buffer loads to LDS, 19 of one kilobyte each), two planes ahead; the buffer of a plane
+// is fixed at compile time by its phase, so that no read waits for a load into another.
+// Bank conflicts: see quad_lane; the strides W1 to W3 (4 mod 8) put the two rows of a write
+// pass on different chunks.  Against the kernel this one replaced (8 waves, each with all four
+// stages in 228 registers; 412 VALU instructions per SIMD and 304 reads per plane), on one box:
+// 16 x 128^3 246 -> 199 us, 16 x 384^3 6320 -> 5150 us per step.  Measured and dropped: loads
+// three planes ahead, the loads or the stores later in the plane, wave priorities by role (no
+// change); reads in the order of consecutive lanes (+2 %); scheduling left to the compiler
+// (+3 %); plain instead of non-temporal stores (+6 %).
 struct QuadCfg {
-    static constexpr int TX = 32, TY = 32, NT = 512, VW = 22;
-    static constexpr int W0 = 54, W1 = 54, W2 = 54, W3 = 38;  // strides of P0..P3
-    static constexpr int WQ = 38, HQ = 34;                     // Q4: stage 4's region + spare rows
-    static constexpr int VW0 = 27;                             // lanes per row of P0's loader
+    static constexpr int TX = 32, TY = 32;
+    static constexpr int NT = 512;        // the tile descriptor's thread count (sp_prop_set_tile)
+    static constexpr int WAVES = 12;      // the launch's waves
+    static constexpr int W0 = 50, W1 = 44, W2 = 44, W3 = 36;  // strides of the planes q, v1, v2, v3
+    static constexpr int H0 = 48, H1 = 44, H2 = 40, H3 = 36;  // their rows
+    static constexpr int LOADS = (W0 / 2 * H0 + 63) / 64;     // wave loads of a q plane
 };
+static_assert(QuadCfg::W1 % 8 == 4 && QuadCfg::W2 % 8 == 4 && QuadCfg::W3 % 8 == 4,
+              "two rows of a write pass on different chunks");
+static_assert(QuadCfg::LOADS > 16 && QuadCfg::LOADS <= 19, "two loads by waves 0-7 and a third by waves 0-2");
 
-template <int S>
-struct QuadMap {
-    using G = Geo<QuadCfg::TX, QuadCfg::TY, S>;
-    static constexpr int U = G::WO / 2;  // blocks per row = block rows
-    static constexpr int VW = QuadCfg::VW, SLOTS = VW * U;
-    static constexpr int WIN = S == 1 ? QuadCfg::W0 : S == 2 ? QuadCfg::W1 : QuadCfg::W2;
-    static constexpr int WOUT = S == 1 ? QuadCfg::W1 : S == 2 ? QuadCfg::W2 : QuadCfg::W3;
-    static_assert(G::WO == G::HOo && U <= VW && SLOTS <= QuadCfg::NT, "one pass of square blocks");
-    static_assert((WIN - VW) % 16 == 0 && (WOUT - VW) % 16 == 0, "conflict-free plane strides");
-    static_assert(WIN >= G::WI && WOUT >= G::WO, "strides cover the regions");
-    static_assert(WIN >= 2 * VW + 4, "spare lanes read inside the padded rows");
-    // block of slot g: column 2*ux and rows 2*uy, 2*uy + 1 of the output region; ux >= U
-    // marks a spare lane; lanes past the last slot repeat it (and write nothing)
-    __device__ static void at(int g, int& ux, int& uy)
-    {
-        g = min(g, SLOTS - 1);
-        uy = g / VW;
-        ux = g % VW;
-    }
-    __device__ static bool live(int g)
-    {
-        int ux, uy;
-        at(g, ux, uy);
-        return ux < U;
-    }
-    __device__ static int centre(int g)  // first row's centre in the input plane
-    {
-        int ux, uy;
-        at(g, ux, uy);
-        return (2 * uy + 2) * WIN + 2 * ux + 2;
-    }
-    __device__ static int out(int g)
-    {
-        int ux, uy;
-        at(g, ux, uy);
-        return 2 * uy * WOUT + 2 * ux;
-    }
-};
+// Lane l's place in the order above, within its wave.  The LDS serves a ds_read_b128 in four
+// passes of 16 lanes, but not of 16 consecutive ones: lanes 0-3, 12-15, 20-23, 24-27 share a
+// pass, then 4-7, 8-11, 16-19, 28-31, and the same in the upper half (measured: rows of 16
+// consecutive lanes take 8.3 cycles per wave at strides of 50 chunks, this order 5.2 at any
+// stride).  The places make every pass one group of 16 blocks.
+__device__ __forceinline__ int quad_lane(int l) { return (l & 32) + ((0x73261540 >> (l & 28)) & 7) * 4 + (l & 3); }
 
-// One stage at one plane for a 2x2 block; point p = 2 f + e (row f, column e).  Each group
-// of LDS reads is issued at raised wave priority: of the two waves sharing a SIMD, the one
-// about to wait on LDS gets its reads out first while the other computes (-3 to -4 % per
-// step at 16 x 128^3, 8 x 160^3, 24 x 96^3).
-template <int S, int R>
-__device__ __forceinline__ void quad_step(const double* __restrict__ P, const StarW<double>& w, double (&acc)[4][4],
-                                          double (&done)[4], d2 (&cen)[2])
+// Block q of the order above, relative to the tile's first block.
+__device__ __forceinline__ void quad_block(int q, int& bx, int& by)
 {
-    constexpr int W = QuadMap<S>::WIN;
-    constexpr int sm2 = (R + 2) & 3, sm1 = (R + 3) & 3, s0 = R & 3, sp1 = (R + 1) & 3;
-    const double* c = P + QuadMap<S>::centre((int)threadIdx.x);
-    double ax[4];
+    if (q < 256) {
+        bx = q & 15;
+        by = q >> 4;
+    } else if (q < 448) {
+        const int d = (q - 192) >> 6, g = ((q & 63) >> 4), i = q & 15;  // ring 1..3; above, below, two halves beside
+        if (g < 2) {
+            bx = i;
+            by = g ? 15 + d : -d;
+        } else {
+            bx = i < 8 ? -d : 15 + d;
+            by = 8 * (g - 2) + (i & 7);
+        }
+    } else {
+        const int i = min(q - 448, 11);  // lanes past the last block repeat it (and write nothing)
+        if (i < 4) {
+            bx = i & 1 ? 16 : -1;
+            by = i & 2 ? 16 : -1;
+        } else {
+            const int j = i - 4, far = j & 1;  // one of (-2, -1), (-1, -2) mirrored to each corner
+            const int ax = far ? 1 : 2, ay = far ? 2 : 1;
+            bx = j & 2 ? 15 + ax : -ax;
+            by = j & 4 ? 15 + ay : -ay;
+        }
+    }
+}
+
+// One stage on a 2x2 block, in parts, so that the reads of one part are in flight during the
+// arithmetic of another.  a: the running sums of one plane's four points, point 2 f + e in row f,
+// column e; c: the block's first centre in an LDS plane (row stride W); u: a plane's centres.
+// A point's terms come in the order z-2, z-1, centre, x, y, z+1, z+2.
+
+__device__ __forceinline__ void quad_fence() { __builtin_amdgcn_sched_barrier(0); }
+// Holds the arithmetic on a there: without it the compiler moves reads past arithmetic, which
+// carries no order of its own, and the values in flight no longer fit the registers.
+__device__ __forceinline__ void quad_hold(double (&a)[4])
+{
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+    __builtin_amdgcn_sched_barrier(0);
+}
+// starts the sums of plane p with the centres of planes p-2 and p-1
+__device__ __forceinline__ void quad_start(double (&a)[4], const StarW<double>& w, const d2 (&um2)[2],
+                                           const d2 (&um1)[2])
+{
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
-        // centres and x neighbours of row f, and the z sums
-        __builtin_amdgcn_s_setprio(1);
-        const d2 C = *(const d2*)(c + f * W), Lx = *(const d2*)(c + f * W - 2), Rx = *(const d2*)(c + f * W + 2);
-        __builtin_amdgcn_s_setprio(0);
-        cen[f] = C;
-        const double u[2] = {C.x, C.y};
+        a[2 * f] = fmaT(w.zm1, um1[f].x, w.zm2 * um2[f].x);
+        a[2 * f + 1] = fmaT(w.zm1, um1[f].y, w.zm2 * um2[f].y);
+    }
+}
+template <int W>
+__device__ __forceinline__ void quad_read_c(const double* __restrict__ c, d2 (&u)[2])
+{
+    u[0] = *(const d2*)c;
+    u[1] = *(const d2*)(c + W);
+}
+// centre and x neighbours (the pairs beside the block's two rows)
+template <int W>
+__device__ __forceinline__ void quad_read_x(const double* __restrict__ c, d2 (&x)[4])
+{
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        x[2 * f] = *(const d2*)(c + f * W - 2);
+        x[2 * f + 1] = *(const d2*)(c + f * W + 2);
+    }
+}
+__device__ __forceinline__ void quad_x(double (&a)[4], const StarW<double>& w, const d2 (&u)[2], const d2 (&x)[4])
+{
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        const d2 C = u[f], Lx = x[2 * f], Rx = x[2 * f + 1];
+        const double c[2] = {C.x, C.y};
         const double xm2[2] = {Lx.x, Lx.y}, xm1[2] = {Lx.y, C.x}, xp1[2] = {C.y, Rx.x}, xp2[2] = {Rx.x, Rx.y};
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const int p = 2 * f + e;
-            done[p] = fmaT(w.zp2, u[e], acc[p][sm2]);
-            acc[p][sm2] = w.zm2 * u[e];
-            acc[p][sm1] = fmaT(w.zp1, u[e], acc[p][sm1]);
-            acc[p][sp1] = fmaT(w.zm1, u[e], acc[p][sp1]);
-            double a = fmaT(w.c, u[e], acc[p][s0]);
-            a = fmaT(w.xm2, xm2[e], a);
-            a = fmaT(w.xm1, xm1[e], a);
-            a = fmaT(w.xp1, xp1[e], a);
-            ax[p] = fmaT(w.xp2, xp2[e], a);
+            double s = fmaT(w.c, c[e], a[2 * f + e]);
+            s = fmaT(w.xm2, xm2[e], s);
+            s = fmaT(w.xm1, xm1[e], s);
+            s = fmaT(w.xp1, xp1[e], s);
+            a[2 * f + e] = fmaT(w.xp2, xp2[e], s);
         }
-        __builtin_amdgcn_sched_barrier(0);
     }
-    {
-        // y neighbours: rows y-2, y-1, y+2, y+3 and the two centre rows
-        __builtin_amdgcn_s_setprio(1);
-        const d2 Ym2 = *(const d2*)(c - 2 * W), Ym1 = *(const d2*)(c - W);
-        const d2 Yp2 = *(const d2*)(c + 2 * W), Yp3 = *(const d2*)(c + 3 * W);
-        __builtin_amdgcn_s_setprio(0);
-        const double r[6][2] = {{Ym2.x, Ym2.y}, {Ym1.x, Ym1.y}, {cen[0].x, cen[0].y},
-                                {cen[1].x, cen[1].y}, {Yp2.x, Yp2.y}, {Yp3.x, Yp3.y}};
+    quad_hold(a);
+}
+// y neighbours: rows y-2, y-1, y+2, y+3 (the block's own rows are the centres)
+template <int W>
+__device__ __forceinline__ void quad_read_y(const double* __restrict__ c, d2 (&y)[4])
+{
+    y[0] = *(const d2*)(c - 2 * W);
+    y[1] = *(const d2*)(c - W);
+    y[2] = *(const d2*)(c + 2 * W);
+    y[3] = *(const d2*)(c + 3 * W);
+}
+__device__ __forceinline__ void quad_y(double (&a)[4], const StarW<double>& w, const d2 (&u)[2], const d2 (&y)[4])
+{
+    const double r[6][2] = {{y[0].x, y[0].y}, {y[1].x, y[1].y}, {u[0].x, u[0].y},
+                            {u[1].x, u[1].y}, {y[2].x, y[2].y}, {y[3].x, y[3].y}};
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+    for (int f = 0; f < 2; ++f)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                // row y+f: neighbours at rows (y+f) -2, -1, +1, +2 = r[f], r[f+1], r[f+3], r[f+4]
-                double a = w.ym2 * r[f][e];
-                a = fmaT(w.ym1, r[f + 1][e], a);
-                a = fmaT(w.yp1, r[f + 3][e], a);
-                a = fmaT(w.yp2, r[f + 4][e], a);
-                acc[2 * f + e][s0] = ax[2 * f + e] + a;
-            }
+        for (int e = 0; e < 2; ++e) {
+            // row y+f: neighbours at rows (y+f) -2, -1, +1, +2 = r[f], r[f+1], r[f+3], r[f+4]
+            double s = w.ym2 * r[f][e];
+            s = fmaT(w.ym1, r[f + 1][e], s);
+            s = fmaT(w.yp1, r[f + 3][e], s);
+            s = fmaT(w.yp2, r[f + 4][e], s);
+            a[2 * f + e] += s;
+        }
+    quad_hold(a);
+}
+// adds the centres of plane p+1
+__device__ __forceinline__ void quad_next(double (&a)[4], const StarW<double>& w, const d2 (&u)[2])
+{
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        a[2 * f] = fmaT(w.zp1, u[f].x, a[2 * f]);
+        a[2 * f + 1] = fmaT(w.zp1, u[f].y, a[2 * f + 1]);
     }
-    __builtin_amdgcn_sched_barrier(0);
+    quad_hold(a);
+}
+// adds the centres of plane p+2 and gives the stage's result q + f * sum
+__device__ __forceinline__ void quad_done(d2 (&v)[2], double f, const double (&a)[4], const StarW<double>& w,
+                                          const d2 (&u)[2], const d2 (&q)[2])
+{
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+        v[r] = d2{fmaT(f, fmaT(w.zp2, u[r].x, a[2 * r]), q[r].x), fmaT(f, fmaT(w.zp2, u[r].y, a[2 * r + 1]), q[r].y)};
 }
 
-// Global byte offsets of the two rows of slot g's block for stage S (periodic images).
-template <int S>
-__device__ __forceinline__ void quad_offsets(int (&q)[2], int x0, int y0, int ni, int nj, int sj)
+template <int W>
+__device__ __forceinline__ void quad_write(double* c, const d2 (&v)[2])
 {
-    using G = Geo<QuadCfg::TX, QuadCfg::TY, S>;
-    int ux, uy;
-    QuadMap<S>::at((int)threadIdx.x, ux, uy);
-    const int gx = pmod(x0 - G::HO + 2 * ux, ni);
+    *(d2*)c = v[0];
+    *(d2*)(c + W) = v[1];
+}
+
+template <int N>
+__device__ __forceinline__ void quad_zero(double (&acc)[N][4])
+{
 #pragma unroll
-    for (int f = 0; f < 2; ++f) q[f] = (gx + pmod(y0 - G::HO + 2 * uy + f, nj) * sj) * 8;
+    for (int j = 0; j < N; ++j) acc[j][0] = acc[j][1] = acc[j][2] = acc[j][3] = 0.;
+}
+
+// Waits until at most N of this wave's vector-memory accesses are outstanding (they complete
+// in the order of issue).
+template <int N>
+__device__ __forceinline__ void vm_wait() { __builtin_amdgcn_s_waitcnt(0x0F70 | N); }
+
+// Workgroup barrier for LDS data: this wave's LDS accesses are complete before it, but for the
+// last N issued (reads of planes that nobody writes next), and none moves across it.  Unlike __syncthreads it leaves loads into LDS in flight (vm_wait before it
+// for those that another wave reads next).
+template <int N = 0>
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_s_waitcnt(0xC07F | N << 8);  // lgkmcnt(N)
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 __device__ __forceinline__ void rk4_quad_body(const FusedArgs& a, const int bid)
 {
-    constexpr int NT = QuadCfg::NT, TX = QuadCfg::TX, TY = QuadCfg::TY;
-    using G1 = Geo<TX, TY, 1>;
-    using G4 = Geo<TX, TY, 4>;
-    using PM4 = PairMap<TX, TY, 4, NT>;
-    static_assert(PM4::M == 1 && PM4::VW == 16, "stage 4: one pass, one row per 16-lane group");
-    constexpr int H0 = G1::HI;                         // rows of the q plane incl. halo
-    constexpr int SLOTS0 = QuadCfg::VW0 * H0;          // loader slots (cols >= WI/2 fill padding)
-    constexpr int M0 = (SLOTS0 + NT - 1) / NT;
-    static_assert(QuadCfg::VW0 * 2 == QuadCfg::W0, "loader slots fill the q plane's rows contiguously");
-    constexpr int W0 = QuadCfg::W0, W1 = QuadCfg::W1, W2 = QuadCfg::W2, W3 = QuadCfg::W3, WQ = QuadCfg::WQ;
+    using Q = QuadCfg;
+    constexpr int W0 = Q::W0, W1 = Q::W1, W2 = Q::W2, W3 = Q::W3;
+    // one array per buffer: reads of one never alias the loads into another
+    __shared__ __attribute__((aligned(16))) double P0a[Q::H0 * W0];
+    __shared__ __attribute__((aligned(16))) double P0b[Q::H0 * W0];
+    __shared__ __attribute__((aligned(16))) double P0c[Q::H0 * W0];
+    __shared__ __attribute__((aligned(16))) double P0d[Q::H0 * W0];
+    __shared__ __attribute__((aligned(16))) double P1[2][Q::H1 * W1];
+    __shared__ __attribute__((aligned(16))) double P2[2][Q::H2 * W2];
+    __shared__ __attribute__((aligned(16))) double P3[2][Q::H3 * W3];
+    const auto P0 = [&](auto Rc) -> double* {
+        constexpr int R = decltype(Rc)::value & 3;
+        if constexpr (R == 0) return P0a;
+        else if constexpr (R == 1) return P0b;
+        else if constexpr (R == 2) return P0c;
+        else return P0d;
+    };
 
-    // q planes of even and odd phase (chunks start on even planes): two arrays, so the
-    // compiler sees that stage 1's reads of one never alias the load into the other
-    __shared__ __attribute__((aligned(16))) double P0a[H0 * W0];
-    __shared__ __attribute__((aligned(16))) double P0b[H0 * W0];
-    __shared__ __attribute__((aligned(16))) double P1[2][Geo<TX, TY, 2>::HI * W1];
-    __shared__ __attribute__((aligned(16))) double P2[2][Geo<TX, TY, 3>::HI * W2];
-    __shared__ __attribute__((aligned(16))) double P3[2][G4::HI * W3];
-    __shared__ __attribute__((aligned(16))) double Q4[2][QuadCfg::HQ * WQ];
-
-    const int tid = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int v = quad_lane(lane);
     const int ni = a.ni, nj = a.nj, nk = a.nk;
     const int tile = bid % a.tiles;
     const int chunk = (bid / a.tiles) % a.chunks;
     const int slice = bid / (a.tiles * a.chunks);
-    const int x0 = (tile % a.tiles_x) * TX, y0 = (tile / a.tiles_x) * TY;
+    const int x0 = (tile % a.tiles_x) * Q::TX, y0 = (tile / a.tiles_x) * Q::TY;
     const int z0 = chunk * a.kchunk;
     const int zend = min(z0 + a.kchunk, nk);
     const __amdgpu_buffer_rsrc_t rin = make_rsrc((const double*)a.in.p + slice * a.in.slice, a.in_bytes);
@@ -1204,163 +1289,253 @@ __device__ __forceinline__ void rk4_quad_body(const FusedArgs& a, const int bid)
     const int isj = (int)a.in.sj, osj = (int)a.out.sj;
     const StarW<double> w = a.cdev ? load_w<double>(a.cdev[slice]) : load_w<double>(a.c);
 
-    // q plane loader: VW0 lanes per row; lanes past the row's 24 pairs load the periodic
-    // continuation into the row's padding (never read), which keeps the writes conflict-free
-    // slot g of the loader is P0 element 2 g: wave w's m-th load fills slots
-    // m NT + 64 w .. + 63, one contiguous kilobyte
-    const int wave = tid >> 6;
-    int off0[M0], dst0[M0];
-#pragma unroll
-    for (int m = 0; m < M0; ++m) {
-        const int g = min(tid + m * NT, SLOTS0 - 1);
-        const int col = g % QuadCfg::VW0, row = g / QuadCfg::VW0;
-        off0[m] = (pmod(x0 - 8 + 2 * col, ni) + pmod(y0 - 8 + row, nj) * isj) * 8;
-        dst0[m] = row * W0 + 2 * col;
-    }
-    const auto wr0 = [&](int m) { return m < M0 - 1 || tid + m * NT < SLOTS0; };  // loader tail: no write
-    int q2[2], q3[2];
-    quad_offsets<2>(q2, x0, y0, ni, nj, isj);
-    quad_offsets<3>(q3, x0, y0, ni, nj, isj);
-    const int o1 = QuadMap<1>::out(tid), o2 = QuadMap<2>::out(tid), o3 = QuadMap<3>::out(tid);
-    static_assert(QuadMap<1>::U == QuadCfg::VW, "stage 1 has no spare lanes");
-    // lanes past a stage's last slot repeat it and write nothing (several lanes writing one
-    // LDS address serialise; reads of one address are a broadcast)
-    const bool live1 = tid < QuadMap<1>::SLOTS;
-    const bool live2 = tid < QuadMap<2>::SLOTS && QuadMap<2>::live(tid);
-    const bool live3 = tid < QuadMap<3>::SLOTS && QuadMap<3>::live(tid);
-    int wq;  // stage 3's block in Q4 (stage 4's region); blocks outside it go to spare cells
-    {
-        int ux, uy;
-        QuadMap<3>::at(tid, ux, uy);
-        int qx = 2 * ux - 2, qy = 2 * uy - 2;
-        if (qx < 0) qx = G4::WO + 2;  // spare columns G4::WO .. WQ-1
-        if (qy < 0) qy = G4::HOo;     // spare rows G4::HOo .. HQ-1
-        wq = qy * WQ + qx;
-    }
-    int o4, r4;
-    {
-        int ax, by;
-        PM4::at(tid, ax, by);
-        o4 = (pmod(x0 + ax, ni) + pmod(y0 + by, nj) * osj) * 8;  // periodic image for partial tiles
-        r4 = by * WQ + ax;
-    }
+    // Iteration t: stage 1's z sums take q(t) and complete v1(t-2), its x and y sums q(t-1),
+    // whose neighbours were read at the end of iteration t-1; stage 2's z sums take v1(t-2) at
+    // once and complete v2(t-4), its x and y sums v1(t-3), written in iteration t-1; stage 3
+    // takes v2(t-5) and completes v3(t-7); stage 4 takes v3(t-8) and completes q'(t-10).  Every
+    // stage runs in every iteration: its first outputs are incomplete and no complete output
+    // reads them.
+    const int tq0 = z0 - 8, tend = zend + 10;
 
-    double acc1[4][4], acc2[4][4], acc3[4][4], acc4[1][2][4];
-    double d1[4], d2v[4], d3[4], d4[1][2];
-    d2 c1[2], c2[2], c3[2], c4[1];
-    d2 qv2[2], qv3[2];
-    d2 r1a[2], r1b[2], r4a, r4b;
+    // Loads of a q plane: load m of wave w fills slots 512 m + 64 w .. + 63 of 16 bytes; slot g
+    // is column pair g % 25 of row g / 25 (the 25th pair is padding).
+    int off0[3];
+    const auto load_offsets = [&] {
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc1[p][j] = acc2[p][j] = acc3[p][j] = 0.;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) acc4[0][e][0] = acc4[0][e][1] = acc4[0][e][2] = acc4[0][e][3] = 0.;
-    r1a[0] = r1a[1] = r1b[0] = r1b[1] = r4a = r4b = d2{0., 0.};
-
-    // Skewed schedule of the pair kernel: iteration t, stage 1: q t -> v1 t-2; stage 2:
-    // v1 t-3 -> v2 t-5; stage 3: v2 t-6 -> v3 t-8; stage 4: v3 t-9 -> q' t-11.
-    const int tq0 = z0 - 8, tq1 = zend + 8;
-    const int tend = zend + 11;
-    {
-        const int zo = wrapz(tq0, nk) * iskb;
-#pragma unroll
-        for (int m = 0; m < M0; ++m)
-            if (wr0(m)) *(d2*)&P0a[dst0[m]] = ld2(rin, off0[m], zo);
-        const int z2 = wrapz(z0 - 8, nk) * iskb, z3 = wrapz(z0 - 6, nk) * iskb;
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-            qv2[f] = ld2(rin, q2[f], z2);
-            qv3[f] = ld2(rin, q3[f], z3);
+        for (int m = 0; m < 3; ++m) {
+            const int g = min(m * 512 + wave * 64 + lane, W0 / 2 * Q::H0 - 1);
+            const int col = g % (W0 / 2), row = g / (W0 / 2);
+            off0[m] = (pmod(x0 - 8 + 2 * col, ni) + pmod(y0 - 8 + row, nj) * isj) * 8;
         }
-    }
-    __syncthreads();
-
-    // One plane at phase R = (t - tq0) & 3.  Every plane issues the same global loads at the
-    // same points, whichever stages are active (a stage's q load fetches the plane it needs
-    // at the next plane, so loads ahead of its first active plane fetch the same values;
-    // past tq1 they fetch valid wrapped planes that no stage reads): the compiler's memory
-    // waits then count them exactly instead of waiting for every load and store of the
-    // previous plane.  Only the output store depends on the plane.
-    auto plane = [&](auto Rc, int t) {
-        constexpr int R = decltype(Rc)::value;
-        const int cur = t & 1, prv = cur ^ 1;
-        double* const P0cur = (R & 1) ? P0b : P0a;  // q(t) (t - tq0 = R mod 4, tq0 even)
-        double* const P0nxt = (R & 1) ? P0a : P0b;
-        __builtin_amdgcn_sched_barrier(0);
-        {
-            // q plane t+1 into P0nxt (read by stage 1 at the next plane; the wait for it
-            // comes before this plane's barrier)
-            const int zo = wrapz(t + 1, nk) * iskb;
-#pragma unroll
-            for (int m = 0; m < M0; ++m)
-                if (wr0(m)) ld2_to_lds(rin, &P0nxt[2 * (m * NT + wave * 64)], off0[m], zo);
+    };
+    const bool third = wave < Q::LOADS - 16, tail = 1024 + wave * 64 + lane < W0 / 2 * Q::H0;
+    const auto load_q = [&](double* P, int p) {  // q plane p
+        const int zo = wrapz(p, nk) * iskb;
+        ld2_to_lds(rin, P + 2 * (wave * 64), off0[0], zo);
+        ld2_to_lds(rin, P + 2 * (512 + wave * 64), off0[1], zo);
+        if (third) {
+            if (tail) ld2_to_lds(rin, P + 2 * (1024 + wave * 64), off0[2], zo);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (t < tq1) {
-            // centres of plane t are q(t); r1b = q(t-2) is the update's q
-            quad_step<1, R & 3>(P0cur, w, acc1, d1, c1);
+    };
+    // before the barrier of a plane: this wave's loads of the previous plane have landed, the
+    // ones of this plane may be in flight
+    const auto wait_q = [&] {
+        if (third) vm_wait<3>();
+        else vm_wait<2>();
+    };
+    using std::integral_constant;
+    // Whole groups of four planes, so that a plane's phase is known at compile time and the
+    // loop has no exits inside; the planes past tend store nothing.
+    const auto stream = [&](auto&& plane) {
+        lds_barrier();
+        for (int t = tq0; t < tend; t += 4) {
+            plane(integral_constant<int, 0>{}, t);
+            plane(integral_constant<int, 1>{}, t + 1);
+            plane(integral_constant<int, 2>{}, t + 2);
+            plane(integral_constant<int, 3>{}, t + 3);
+        }
+    };
+
+    if (wave < 6 || wave == 7) {
+        // ---- stages 1 and 2
+        const int q = wave < 6 ? wave * 64 + v : 448 + v;
+        int bx, by;
+        quad_block(q, bx, by);
+        const int i0 = (2 * by + 8) * W0 + 2 * bx + 8;
+        const int i1 = (2 * by + 6) * W1 + 2 * bx + 6;
+        const int i2 = (2 * by + 4) * W2 + 2 * bx + 4;
+        // wave 7: lanes without a block in a stage write nothing
+        const bool live1 = q < 460, live2 = q < 452;
+        load_offsets();
+        // running sums by plane phase: stage 1's of two planes, stage 2's of three
+        double a1[4][4], a2[4][4];
+        d2 uc[2], qr[4][2];  // v1 of this block; q at lags 1-4 by plane phase
+        d2 x[4], y[4];
+        quad_zero(a1);
+        quad_zero(a2);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) uc[f] = qr[0][f] = qr[1][f] = qr[2][f] = qr[3][f] = d2{0., 0.};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = y[i] = d2{0., 0.};
+        load_q(P0a, tq0);
+        load_q(P0b, tq0 + 1);
+        vm_wait<0>();
+        stream([&](auto Rc, int t) {
+            constexpr int R = decltype(Rc)::value, cur = R & 1, prv = cur ^ 1;
+            constexpr int R1 = (R + 3) & 3, R2 = (R + 2) & 3, R3 = (R + 1) & 3;  // phases of planes t-1, t-2, t-3
+            load_q(P0(integral_constant<int, R + 2>{}), t + 2);
+            const double *const c0 = P0(Rc) + i0, *const c1 = &P1[prv][i1];
+            d2 qc[2], un[2], v2[2];
+            quad_read_c<W0>(c0, qc);
+            quad_start(a1[R1], w, qr[R3], qr[R2]);
+            quad_x(a1[R1], w, qr[R1], x);
+            quad_read_x<W1>(c1, x);
+            quad_fence();
+            quad_y(a1[R1], w, qr[R1], y);
+            quad_read_y<W1>(c1, y);
+            quad_fence();
+            quad_x(a2[R3], w, uc, x);
+            quad_y(a2[R3], w, uc, y);
+            quad_done(un, w.f1, a1[R2], w, qc, qr[R2]);
+            if (live1) quad_write<W1>(&P1[cur][i1], un);
+            quad_fence();
+            quad_done(v2, w.f2, a2[R], w, un, qr[R]);
+            if (live2) quad_write<W2>(&P2[cur][i2], v2);
+            quad_fence();
+            quad_read_x<W0>(c0, x);
+            quad_read_y<W0>(c0, y);
+            quad_fence();
+            quad_next(a1[R1], w, qc);
+            quad_next(a2[R3], w, un);
+            quad_start(a2[R1], w, uc, un);
+            quad_hold(a2[R1]);
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
-                if (live1)
-                    *(d2*)&P1[cur][o1 + f * W1] =
-                        d2{fmaT(w.f1, d1[2 * f], r1b[f].x), fmaT(w.f1, d1[2 * f + 1], r1b[f].y)};
-                r1b[f] = r1a[f];
-                r1a[f] = c1[f];
+                uc[f] = un[f];
+                qr[R][f] = qc[f];
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (t >= tq0 + 5 && t < tq1 + 1) {
-            quad_step<2, (R + 1) & 3>(P1[prv], w, acc2, d2v, c2);
-            if (live2) {
+            wait_q();
+            lds_barrier<8>();
+        });
+        vm_wait<0>();  // no load into LDS outlives the block
+    } else if (wave == 6) {
+        // ---- stage 1 on ring 3, stage 3 on ring 1
+        int bx, by, cx, cy;
+        quad_block(384 + v, bx, by);
+        quad_block(256 + v, cx, cy);
+        const int i0 = (2 * by + 8) * W0 + 2 * bx + 8;
+        const int i1 = (2 * by + 6) * W1 + 2 * bx + 6;
+        const int i2 = (2 * cy + 4) * W2 + 2 * cx + 4;
+        const int i3 = (2 * cy + 2) * W3 + 2 * cx + 2;
+        int q3[2];
 #pragma unroll
-                for (int f = 0; f < 2; ++f)
-                    *(d2*)&P2[cur][o2 + f * W2] =
-                        d2{fmaT(w.f2, d2v[2 * f], qv2[f].x), fmaT(w.f2, d2v[2 * f + 1], qv2[f].y)};
+        for (int f = 0; f < 2; ++f) q3[f] = (pmod(x0 + 2 * cx, ni) + pmod(y0 + 2 * cy + f, nj) * isj) * 8;
+        load_offsets();
+        double a1[4][4], a3[4][4];
+        d2 qr[4][2], vp[2], qe[2], qo[2];  // q at lags 1-4 by plane phase, v2 of the last plane, q at lags 7 and 6
+        d2 x[4], y[4];
+        quad_zero(a1);
+        quad_zero(a3);
+        vp[0] = vp[1] = qe[0] = qe[1] = qo[0] = qo[1] = d2{0., 0.};
+#pragma unroll
+        for (int f = 0; f < 2; ++f) qr[0][f] = qr[1][f] = qr[2][f] = qr[3][f] = d2{0., 0.};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = y[i] = d2{0., 0.};
+        load_q(P0a, tq0);
+        load_q(P0b, tq0 + 1);
+        vm_wait<0>();
+        stream([&](auto Rc, int t) {
+            constexpr int R = decltype(Rc)::value, cur = R & 1, prv = cur ^ 1;
+            constexpr int R1 = (R + 3) & 3, R2 = (R + 2) & 3, R3 = (R + 1) & 3;
+            load_q(P0(integral_constant<int, R + 2>{}), t + 2);
+            const double *const c0 = P0(Rc) + i0, *const c2 = &P2[prv][i2];
+            d2(&qv)[2] = R & 1 ? qo : qe;  // q(t-7)
+            d2 qc[2], vc[2], v1[2], v3[2];
+            quad_read_c<W0>(c0, qc);
+            quad_read_c<W2>(c2, vc);
+            quad_start(a1[R1], w, qr[R3], qr[R2]);
+            quad_x(a1[R1], w, qr[R1], x);
+            quad_read_x<W2>(c2, x);
+            quad_fence();
+            quad_y(a1[R1], w, qr[R1], y);
+            quad_read_y<W2>(c2, y);
+            quad_fence();
+            quad_done(v1, w.f1, a1[R2], w, qc, qr[R2]);
+            quad_write<W1>(&P1[cur][i1], v1);
+            quad_fence();
+            // plane t-5: its phase is R1, t-6's R2, t-7's R3
+            quad_done(v3, w.f3, a3[R3], w, vc, qv);
+            quad_write<W3>(&P3[cur][i3], v3);
+            quad_fence();
+            {
+                const int zo = wrapz(t - 5, nk) * iskb;  // q(t-5): stage 3's q two planes on
+#pragma unroll
+                for (int f = 0; f < 2; ++f) qv[f] = ld2(rin, q3[f], zo);
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        {
-            const int zo = wrapz(t - 4, nk) * iskb;  // q(t-4): stage 2's q at the next plane
+            quad_next(a3[R2], w, vc);
+            quad_x(a3[R1], w, vc, x);
+            quad_y(a3[R1], w, vc, y);
+            quad_read_x<W0>(c0, x);
+            quad_read_y<W0>(c0, y);
+            quad_fence();
+            quad_next(a1[R1], w, qc);
+            quad_start(a3[R], w, vp, vc);
+            quad_hold(a3[R]);
 #pragma unroll
-            for (int f = 0; f < 2; ++f) qv2[f] = ld2(rin, q2[f], zo);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (t >= tq0 + 10 && t < tq1 + 2) {
-            quad_step<3, (R + 2) & 3>(P2[prv], w, acc3, d3, c3);
-            if (live3) {
-#pragma unroll
-                for (int f = 0; f < 2; ++f) {
-                    *(d2*)&P3[cur][o3 + f * W3] =
-                        d2{fmaT(w.f3, d3[2 * f], qv3[f].x), fmaT(w.f3, d3[2 * f + 1], qv3[f].y)};
-                    *(d2*)&Q4[cur][wq + f * WQ] = qv3[f];  // q(t-8) for stage 4
-                }
+            for (int f = 0; f < 2; ++f) {
+                vp[f] = vc[f];
+                qr[R][f] = qc[f];
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        {
-            const int zo = wrapz(t - 7, nk) * iskb;  // q(t-7): stage 3's q at the next plane
+            vm_wait<6>();  // two loads of a q plane and two of q since the last plane's
+            lds_barrier<8>();
+        });
+        vm_wait<0>();
+    } else {
+        // ---- stages 3 and 4
+        int bx, by;
+        quad_block((wave - 8) * 64 + v, bx, by);
+        const int i2 = (2 * by + 4) * W2 + 2 * bx + 4;
+        const int i3 = (2 * by + 2) * W3 + 2 * bx + 2;
+        int q3[2], o4[2];
 #pragma unroll
-            for (int f = 0; f < 2; ++f) qv3[f] = ld2_last(rin, q3[f], zo);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int f = 0; f < 2; ++f) {
+            const int gx = pmod(x0 + 2 * bx, ni), gy = pmod(y0 + 2 * by + f, nj);  // periodic image for partial tiles
+            q3[f] = (gx + gy * isj) * 8;
+            o4[f] = (gx + gy * osj) * 8;
         }
-        if (t >= tq0 + 15) {
-            pair_step<TX, TY, 4, NT, 1, (R + 3) & 3, W3>(P3[prv], w, acc4, d4, c4);
-            const int zp = t - 11;
-            if (zp >= z0 && zp < zend)
-                st2_stream(rout, o4, zp * oskb, d2{fmaT(w.f4, d4[0][0], r4b.x), fmaT(w.f4, d4[0][1], r4b.y)});
-            r4b = r4a;
-            r4a = *(const d2*)&Q4[prv][r4];  // q(t-9)
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    for (int t = tq0; t < tend; t += 4) {
-        plane(std::integral_constant<int, 0>{}, t);
-        if (t + 1 < tend) plane(std::integral_constant<int, 1>{}, t + 1);
-        if (t + 2 < tend) plane(std::integral_constant<int, 2>{}, t + 2);
-        if (t + 3 < tend) plane(std::integral_constant<int, 3>{}, t + 3);
+        double a3[4][4], a4[4][4];
+        d2 yc[2], yp[2], vp[2], qr[4][2];  // v3 of this block and the plane before, v2 before; q at lags 7-10
+        quad_zero(a3);
+        quad_zero(a4);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) yc[f] = yp[f] = vp[f] = qr[0][f] = qr[1][f] = qr[2][f] = qr[3][f] = d2{0., 0.};
+        stream([&](auto Rc, int t) {
+            constexpr int R = decltype(Rc)::value, cur = R & 1, prv = cur ^ 1;
+            constexpr int R1 = (R + 3) & 3, R2 = (R + 2) & 3, R3 = (R + 1) & 3;
+            const double *const c2 = &P2[prv][i2], *const c3 = &P3[prv][i3];
+            d2 vc[2], x[4], y[4], qn[2];
+            quad_read_x<W3>(c3, x);
+            quad_read_y<W3>(c3, y);
+            quad_fence();
+            // stage 4 at plane t-8 (phase R; t-9's R1, t-10's R2): the stores outside z0 to zend
+            // go past the field's end and are dropped (issued all the same, so that waits count
+            // loads and stores exactly)
+            const bool st = t >= tq0 + 18 && t < tend;
+            const int zo = st ? (t - 10) * oskb : 0;
+            quad_done(qn, w.f4, a4[R2], w, yc, qr[R2]);
+#pragma unroll
+            for (int f = 0; f < 2; ++f) st2_stream(rout, st ? o4[f] : (int)0x80000000, zo, qn[f]);
+            {
+                const int zq = wrapz(t - 6, nk) * iskb;  // q(t-6): stage 3's q at the next plane
+#pragma unroll
+                for (int f = 0; f < 2; ++f) qr[R2][f] = ld2_last(rin, q3[f], zq);
+            }
+            quad_fence();
+            quad_next(a4[R1], w, yc);
+            quad_x(a4[R], w, yc, x);
+            quad_read_c<W2>(c2, vc);
+            quad_read_x<W2>(c2, x);
+            quad_fence();
+            quad_y(a4[R], w, yc, y);
+            quad_read_y<W2>(c2, y);
+            quad_fence();
+            quad_start(a4[R3], w, yp, yc);
+            quad_hold(a4[R3]);
+#pragma unroll
+            for (int f = 0; f < 2; ++f) yp[f] = yc[f];
+            // stage 3 at plane t-5 (phase R1; t-6's R2, t-7's R3)
+            quad_done(yc, w.f3, a3[R3], w, vc, qr[R3]);
+            quad_write<W3>(&P3[cur][i3], yc);
+            quad_fence();
+            quad_next(a3[R2], w, vc);
+            quad_x(a3[R1], w, vc, x);
+            quad_y(a3[R1], w, vc, y);
+            quad_start(a3[R], w, vp, vc);
+            quad_hold(a3[R]);
+#pragma unroll
+            for (int f = 0; f < 2; ++f) vp[f] = vc[f];
+            lds_barrier();
+        });
     }
 }
 
@@ -1377,7 +1552,7 @@ __global__ void __launch_bounds__(NT) k_rk4_fused_pair(FusedArgs a)
     rk4_pair_body<SI, SO, T, TX, TY, NT>(a, xcd_block(blockIdx.x, gridDim.x));
 }
 
-__global__ void __launch_bounds__(QuadCfg::NT) k_rk4_fused_quad(FusedArgs a)
+__global__ void __launch_bounds__(QuadCfg::WAVES * 64) k_rk4_fused_quad(FusedArgs a)
 {
     rk4_quad_body(a, xcd_block(blockIdx.x, gridDim.x));
 }
@@ -1420,7 +1595,7 @@ __global__ void __launch_bounds__(NT) k_rk4_fused_pair_grouped(GroupArgs g)
     rk4_pair_body<SI, SO, T, TX, TY, NT>(*(const FusedArgs*)rec, bid - g.first[e]);
 }
 
-__global__ void __launch_bounds__(QuadCfg::NT) k_rk4_fused_quad_grouped(GroupArgs g)
+__global__ void __launch_bounds__(QuadCfg::WAVES * 64) k_rk4_fused_quad_grouped(GroupArgs g)
 {
     const int bid = xcd_block(blockIdx.x, gridDim.x);
     const int e = group_entry(g, bid);
@@ -1472,9 +1647,6 @@ int fill_args(FusedArgs& a, const FusedStep& st, const FusedTile& tile, View in,
     a.nj = st.nj;
     a.nk = st.nk;
     a.kchunk = tile.kchunk > 0 ? min(tile.kchunk, st.nk) : st.nk;
-    // the 2x2 kernel's chunks start on even planes (its q-plane buffers alternate by plane
-    // parity); the chunking does not change the results
-    if (tile.variant == SP_KERNEL_QUAD && a.kchunk < st.nk && (a.kchunk & 1)) a.kchunk += 1;
     a.tiles_x = (st.ni + tile.tx - 1) / tile.tx;
     const int tiles_y = (st.nj + tile.ty - 1) / tile.ty;
     a.tiles = a.tiles_x * tiles_y;
@@ -1534,7 +1706,7 @@ int launch_quad(hipStream_t s, const FusedStep& st, const FusedTile& tile, View 
              "fused RK4 (2x2): unsupported tile shape");
     FusedArgs a;
     SP_TRY(fill_args(a, st, tile, in, out, 8, 8));
-    hipLaunchKernelGGL(k_rk4_fused_quad, dim3(nblocks_of(a, st.nslices)), dim3(QuadCfg::NT), 0, s, a);
+    hipLaunchKernelGGL(k_rk4_fused_quad, dim3(nblocks_of(a, st.nslices)), dim3(QuadCfg::WAVES * 64), 0, s, a);
     SP_HIP(hipGetLastError());
     return SP_OK;
 }
@@ -1647,7 +1819,7 @@ int launch_rk4_grouped(hipStream_t s, const FusedTile& tile, int in_dtype, int o
         SP_CHECK(in_dtype == SP_F64 && out_dtype == SP_F64, SP_ERR_UNSUPPORTED, "grouped 2x2 kernel is FP64 only");
         SP_CHECK(tile.tx == QuadCfg::TX && tile.ty == QuadCfg::TY && tile.nt == QuadCfg::NT, SP_ERR_UNSUPPORTED,
                  "grouped fused RK4 (2x2): unsupported tile shape");
-        hipLaunchKernelGGL(k_rk4_fused_quad_grouped, dim3((unsigned)nblocks), dim3(QuadCfg::NT), 0, s, g);
+        hipLaunchKernelGGL(k_rk4_fused_quad_grouped, dim3((unsigned)nblocks), dim3(QuadCfg::WAVES * 64), 0, s, g);
         SP_HIP(hipGetLastError());
         return SP_OK;
     }

@@ -1,0 +1,46 @@
+"""Fused RK4 kernels at the edges of their tiles and k chunks: widths below, at and past a
+tile, the thinnest k extent, chunks of a plane count that is no multiple of the planes a loop
+turn takes, strided batches.  Every FP64 variant evaluates each point with the same operation
+sequence, so the scalar kernel's result is the reference, bit for bit; the oracle bounds both
+(1e-12 of the largest value, the bound stated for the fused kernels)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+import oracle as O  # noqa: E402
+
+C3 = (1.0, -0.5, 0.25)
+
+
+@pytest.fixture(scope="module")
+def sp():
+    import stencilparareal_amd as spm
+    from stencilparareal_amd import field
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    field.Context.default(0)
+    return spm
+
+
+def run(sp, shape, variant, tile, kchunk, steps=3, nufreq=0.0):
+    ni, nj, nk = shape
+    q0 = np.random.default_rng(ni * 100 + nj + nk).standard_normal((nk, nj, ni))
+    conv = sp.Convection(ni, nj, nk, 1. / 32, 0.02, nufreq, *C3)
+    conv.set_tile(*tile, kchunk, variant=variant)
+    a, b = conv.field(), conv.field()
+    a.set(q0)
+    conv.DoRK4(a, b, 0.0, 1e-4, steps)
+    return q0, b.get()
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 8), (8, 8, 8), (30, 31, 9), (32, 32, 10), (34, 33, 11), (66, 2, 17), (96, 64, 16)],
+                         ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("kchunk", [0, 1, 3, 6])
+def test_quad_kernel_edges(sp, shape, kchunk):
+    q0, ref = run(sp, shape, "scalar", (32, 16, 512), 0)
+    _, got = run(sp, shape, "quad", (32, 32, 512), kchunk)
+    assert np.array_equal(got, ref)
+    exact = O.OConvection(*shape, 1. / 32, 0.02, 0.0, *C3).rk4(q0, 0.0, 1e-4, 3)
+    assert np.abs(got - exact).max() <= 1e-12 * np.abs(exact).max()
