@@ -121,12 +121,13 @@ int sp_prop_set_path(sp_prop* p, int path);
  * kchunk planes per block (0: whole k extent).  variant SP_KERNEL_AUTO restores the
  * built-in choice.  Compiled shapes: scalar {32x32x1024, 32x24x1024, 24x24x1024,
  * 32x16x512, 16x16x256}, pair {32x32x512, 32x16x512, 16x16x256}, quad {32x32x512}
- * (its blocks run 768 threads; the built-in choice for FP64 launches of 256 or more
- * blocks; FP32 / BF16 storage takes the pair kernel in its place), split {32x32x512,
- * 32x16x512, 32x16x256, 16x16x256}.  The split variant (FP64 fields, even ni) runs each
+ * (its blocks run 768 threads; the built-in choice for FP64, but for fields of few bricks;
+ * FP32 / BF16 storage takes the pair kernel in its place), split {32x32x512,
+ * 32x16x512, 32x16x256, 16x16x256, 16x16x384}.  The split variant (FP64 fields) runs each
  * step as two launches through a work field the propagator allocates (8 bytes per point
  * of the batch) when the tile is chosen; its results equal the other FP64 variants' bit
- * for bit.  Grouped batches (sp_batch_*) and sp_do_rk4_noalloc run the built-in FP64
+ * for bit.  Its shape 16x16x384 computes bricks of 16x16x8 points (whatever kchunk says), on
+ * any sizes and strides; the other shapes need an even ni.  Grouped batches (sp_batch_*) and sp_do_rk4_noalloc run the built-in FP64
  * choice in its place. */
 int sp_prop_set_tile(sp_prop* p, int variant, int tx, int ty, int nthreads, int kchunk);
 /* The fused-kernel tile sp_do_rk4 (nslices = 1) or sp_do_rk4_batched (nslices > 1) will

@@ -576,8 +576,9 @@ int sp_prop_get_tile(const sp_prop* p, int nslices, int f64, int* variant, int* 
     SP_CHECK(nslices >= 1, SP_ERR_INVALID, "sp_prop_get_tile: nslices < 1");
     FusedTile t = pick_tile(p, nslices, f64 ? 1 : 0);
     // the pair kernel needs an even x extent (as every layout then has even strides); the
-    // 2x2 and split kernels also FP64
-    if (t.variant != SP_KERNEL_SCALAR && (p->ni % 2 != 0 || (!f64 && t.variant != SP_KERNEL_PAIR)))
+    // 2x2 and split kernels also FP64 (the split kernel's bricks FP64 only)
+    const bool any_ni = t.variant == SP_KERNEL_SCALAR || (f64 && fused_tile_brick(t));
+    if (!any_ni && (p->ni % 2 != 0 || (!f64 && t.variant != SP_KERNEL_PAIR)))
         t = FusedTile{32, 16, 512, t.kchunk, SP_KERNEL_SCALAR};
     if (variant) *variant = t.variant;
     if (tx) *tx = t.tx;
@@ -674,7 +675,7 @@ int sp_do_rk4_noalloc(sp_prop* p, const sp_layout* lin, const void* in, const sp
     FusedTile tile = pick_tile(p, 1, 1);
     // the split steps need a second intermediate field: the built-in one-launch tile instead
     // (the same result bit for bit)
-    if (tile.variant == SP_KERNEL_SPLIT) tile = default_tile(p->ni, p->nj, p->nk, 1, 1);
+    if (tile.variant == SP_KERNEL_SPLIT) tile = default_tile(p->ni, p->nj, p->nk, 1, 1, true);
     // out and A alternate so the last step lands in out; in place (in == out), the first
     // step must not write in, so an odd count ends in A and is copied to out
     View src = vin;

@@ -241,11 +241,11 @@ __device__ __forceinline__ void stage_qload(T (&qv)[M], __amdgpu_buffer_rsrc_t r
 
 // Blocks are handed to the 8 XCDs round-robin (block b runs on XCD b % 8).  Renumber so
 // that each XCD receives a contiguous range of tiles: neighbouring tiles, which read each
-// other's halo columns, then share one L2.
+// other's halo columns, then share one L2.  (The first n % 8 XCDs get one block more.)
 __device__ __forceinline__ int xcd_block(int b, int n)
 {
-    if (n % 8 != 0) return b;
-    return (b % 8) * (n / 8) + b / 8;
+    const int x = b % 8, r = n % 8;
+    return x * (n / 8) + min(x, r) + b / 8;
 }
 
 template <typename SI, typename SO, typename T, int TX, int TY, int NT>
@@ -1158,6 +1158,7 @@ __device__ __forceinline__ void quad_read_x(const double* __restrict__ c, d2 (&x
         x[2 * f + 1] = *(const d2*)(c + f * W + 2);
     }
 }
+template <bool HOLD = true>
 __device__ __forceinline__ void quad_x(double (&a)[4], const StarW<double>& w, const d2 (&u)[2], const d2 (&x)[4])
 {
 #pragma unroll
@@ -1174,7 +1175,7 @@ __device__ __forceinline__ void quad_x(double (&a)[4], const StarW<double>& w, c
             a[2 * f + e] = fmaT(w.xp2, xp2[e], s);
         }
     }
-    quad_hold(a);
+    if constexpr (HOLD) quad_hold(a);
 }
 // y neighbours: rows y-2, y-1, y+2, y+3 (the block's own rows are the centres)
 template <int W>
@@ -1185,6 +1186,7 @@ __device__ __forceinline__ void quad_read_y(const double* __restrict__ c, d2 (&y
     y[2] = *(const d2*)(c + 2 * W);
     y[3] = *(const d2*)(c + 3 * W);
 }
+template <bool HOLD = true>
 __device__ __forceinline__ void quad_y(double (&a)[4], const StarW<double>& w, const d2 (&u)[2], const d2 (&y)[4])
 {
     const double r[6][2] = {{y[0].x, y[0].y}, {y[1].x, y[1].y}, {u[0].x, u[0].y},
@@ -1200,9 +1202,10 @@ __device__ __forceinline__ void quad_y(double (&a)[4], const StarW<double>& w, c
             s = fmaT(w.yp2, r[f + 4][e], s);
             a[2 * f + e] += s;
         }
-    quad_hold(a);
+    if constexpr (HOLD) quad_hold(a);
 }
 // adds the centres of plane p+1
+template <bool HOLD = true>
 __device__ __forceinline__ void quad_next(double (&a)[4], const StarW<double>& w, const d2 (&u)[2])
 {
 #pragma unroll
@@ -1210,7 +1213,7 @@ __device__ __forceinline__ void quad_next(double (&a)[4], const StarW<double>& w
         a[2 * f] = fmaT(w.zp1, u[f].x, a[2 * f]);
         a[2 * f + 1] = fmaT(w.zp1, u[f].y, a[2 * f + 1]);
     }
-    quad_hold(a);
+    if constexpr (HOLD) quad_hold(a);
 }
 // adds the centres of plane p+2 and gives the stage's result q + f * sum
 __device__ __forceinline__ void quad_done(d2 (&v)[2], double f, const double (&a)[4], const StarW<double>& w,
@@ -1539,6 +1542,175 @@ __device__ __forceinline__ void rk4_quad_body(const FusedArgs& a, const int bid)
     }
 }
 
+// ---- FP64 step of small fields: bricks, two launches of two stages ---------------------------
+// A small field has too few tiles to fill the chip, and a chunk's walk along k is bound by one
+// plane's latency (0.5-1.2 us) times its planes, most of which fill the pipeline.  Here nothing
+// walks: a block loads the whole input of a 16x16x8 brick of results at once (24x24x16 cells,
+// 80 KB of LDS, two blocks per CU), computes one stage on its 20x20x12 cells (without the
+// corners, 96 2x2 columns x 12 planes over 384 lanes, three planes each), puts the result over
+// the input in LDS and computes the next stage.  Four stages take two launches through the
+// work field of the split step:
+//   launch A: u = q,  v_a = q + f1 L u,  out = q + f2 L v_a   (= v2)
+//   launch B: u = v2, v_a = q + f3 L u,  out = q + f4 L v_a   (= q')
+// with the other kernels' operations in the same order (the same bits).  Any sizes, strides and
+// alignment: PAIR loads and stores 16 bytes, otherwise each cell's two words are loaded by
+// lanes of their own.  Conflict-free planes: 10 columns per row of the first stage and a row
+// pair of 26 chunks (10 mod 16) put consecutive lanes on consecutive chunks across rows.
+struct BrickCfg {
+    static constexpr int BX = 16, BY = 16, BZ = 8, NT = 384;
+    static constexpr int W = 26, H = 24, D = 16, PLANE = W * H;  // the input's cells in LDS
+};
+
+// The base values q of a lane's 2x2 block in N planes, from global memory.
+template <bool PAIR>
+struct BrickCols {
+    int o[2][PAIR ? 1 : 2];  // byte offsets of the block's rows (and columns, if not PAIR)
+    __device__ __forceinline__ void set(int x, int y, int ni, int nj, int sj)
+    {
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int e = 0; e < (PAIR ? 1 : 2); ++e) o[f][e] = (pmod(x + e, ni) + pmod(y + f, nj) * sj) * 8;
+    }
+    __device__ __forceinline__ d2 ld(__amdgpu_buffer_rsrc_t r, int f, int zo) const
+    {
+        if constexpr (PAIR) return ld2(r, o[f][0], zo);
+        else return d2{Buf<double>::ld(r, o[f][0], zo), Buf<double>::ld(r, o[f][1], zo)};
+    }
+    __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, int f, int zo, d2 v) const
+    {
+        if constexpr (PAIR) {
+            st2(r, o[f][0], zo, v);
+        } else {
+            Buf<double>::st(r, o[f][0], zo, v.x);
+            Buf<double>::st(r, o[f][1], zo, v.y);
+        }
+    }
+};
+
+// One stage of a block's column at N consecutive planes; c: its first centre two planes below.
+template <int N>
+__device__ __forceinline__ void brick_stage(d2 (&v)[N][2], const double* __restrict__ c, const StarW<double>& w,
+                                            double f, const d2 (*q)[2])
+{
+    using B = BrickCfg;
+    d2 u[N + 4][2];
+#pragma unroll
+    for (int k = 0; k < N + 4; ++k) quad_read_c<B::W>(c + k * B::PLANE, u[k]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const double* p = c + (j + 2) * B::PLANE;
+        d2 x[4], y[4];
+        double a[4];
+        quad_read_x<B::W>(p, x);
+        quad_read_y<B::W>(p, y);
+        quad_start(a, w, u[j], u[j + 1]);
+        quad_x<false>(a, w, u[j + 2], x);
+        quad_y<false>(a, w, u[j + 2], y);
+        quad_next<false>(a, w, u[j + 3]);
+        quad_done(v[j], f, a, w, u[j + 4], q ? q[j] : u[j + 2]);
+    }
+}
+
+template <bool FIRST, bool PAIR>
+__device__ __forceinline__ void rk4_brick_body(const HalfArgs& h, const int bid)
+{
+    using B = BrickCfg;
+    const FusedArgs& a = h.a;
+    __shared__ __attribute__((aligned(16))) double P[B::D * B::PLANE];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ni = a.ni, nj = a.nj, nk = a.nk;
+    const int tile = bid % a.tiles;
+    const int chunk = (bid / a.tiles) % a.chunks;
+    const int slice = bid / (a.tiles * a.chunks);
+    const int x0 = (tile % a.tiles_x) * B::BX, y0 = (tile / a.tiles_x) * B::BY, z0 = chunk * B::BZ;
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc((const double*)a.in.p + slice * a.in.slice, a.in_bytes);
+    const __amdgpu_buffer_rsrc_t rq = make_rsrc((const double*)h.q.p + slice * h.q.slice, h.q_bytes);
+    const __amdgpu_buffer_rsrc_t rout = make_rsrc((double*)a.out.p + slice * a.out.slice, a.out_bytes);
+    const int iskb = (int)a.in.sk * 8, qskb = (int)h.q.sk * 8, oskb = (int)a.out.sk * 8;
+    const StarW<double> w = a.cdev ? load_w<double>(a.cdev[slice]) : load_w<double>(a.c);
+
+    // The input's planes, each 312 16-byte slots in the order of the cells: waves 0-4 load a
+    // slot per lane, or (not PAIR) four words per lane.
+    if (wave < 5) {
+        constexpr int M = PAIR ? 1 : 4;
+        int off[M];
+        bool in[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int e = PAIR ? 2 * (wave * 64 + lane) : wave * 128 + m * 32 + (lane >> 1);  // cell of the plane
+            in[m] = e < B::PLANE;
+            off[m] = (pmod(x0 - 4 + e % B::W, ni) + pmod(y0 - 4 + e / B::W, nj) * (int)a.in.sj) * 8 +
+                     (PAIR ? 0 : (lane & 1) * 4);
+        }
+#pragma unroll
+        for (int p = 0; p < B::D; ++p) {
+            const int zo = wrapz(z0 - 4 + p, nk) * iskb;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                double* const dst = P + p * B::PLANE + wave * 128 + m * 32;
+                if (in[m]) {
+                    if constexpr (PAIR) ld2_to_lds(rin, dst, off[m], zo);
+                    else
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(rin, (__attribute__((address_space(3))) void*)dst, 4,
+                                                                 off[m], zo, 0, 0);
+                }
+            }
+        }
+    }
+    // first stage: column 96 zg + s of three planes; s in rows of 8, 10 (eight times), 8 blocks
+    const int za = tid / 96, sa = tid % 96;
+    const int by = sa < 8 ? -1 : sa < 88 ? (sa - 8) / 10 : 8;
+    const int bx = sa < 8 ? sa : sa < 88 ? (sa - 8) % 10 - 1 : sa - 88;
+    double* const ca = P + 3 * za * B::PLANE + (2 * by + 4) * B::W + 2 * bx + 4;
+    d2 qa[3][2];
+    if constexpr (!FIRST) {
+        BrickCols<PAIR> col;
+        col.set(x0 + 2 * bx, y0 + 2 * by, ni, nj, (int)h.q.sj);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int f = 0; f < 2; ++f) qa[j][f] = col.ld(rq, f, wrapz(z0 - 2 + 3 * za + j, nk) * qskb);
+    }
+    // second stage: waves 0-3, two planes each
+    const int zb = wave, cx = x0 + 2 * (lane & 7), cy = y0 + 2 * (lane >> 3);
+    d2 qb[2][2];
+    if (wave < 4) {
+        BrickCols<PAIR> col;
+        col.set(cx, cy, ni, nj, (int)h.q.sj);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int f = 0; f < 2; ++f) qb[j][f] = col.ld(rq, f, wrapz(z0 + 2 * zb + j, nk) * qskb);
+    }
+    vm_wait<0>();
+    lds_barrier();
+    d2 va[3][2];
+    if constexpr (FIRST) brick_stage<3>(va, ca, w, w.f1, nullptr);
+    else brick_stage<3>(va, ca, w, w.f3, qa);
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 3; ++j) quad_write<B::W>(ca + (j + 2) * B::PLANE, va[j]);
+    lds_barrier();
+    if (wave < 4) {
+        const double* const cb = P + (2 * zb + 2) * B::PLANE + (2 * (lane >> 3) + 4) * B::W + 2 * (lane & 7) + 4;
+        d2 vb[2][2];
+        brick_stage<2>(vb, cb, w, FIRST ? w.f2 : w.f4, qb);
+        BrickCols<PAIR> col;
+        col.set(cx, cy, ni, nj, (int)a.out.sj);  // periodic image for partial bricks
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int z = z0 + 2 * zb + j;
+            if (z < nk) {
+#pragma unroll
+                for (int f = 0; f < 2; ++f) col.st(rout, f, z * oskb, vb[j][f]);
+            }
+        }
+    }
+}
+
 // One launch over one batch of slices.
 template <typename SI, typename SO, typename T, int TX, int TY, int NT>
 __global__ void __launch_bounds__(NT) k_rk4_fused(FusedArgs a)
@@ -1561,6 +1733,12 @@ template <int TX, int TY, int NT, bool FIRST>
 __global__ void __launch_bounds__(NT) k_rk4_half_pair(HalfArgs h)
 {
     rk4_half_pair_body<TX, TY, NT, FIRST>(h, xcd_block(blockIdx.x, gridDim.x));
+}
+
+template <bool FIRST, bool PAIR>
+__global__ void __launch_bounds__(BrickCfg::NT, 3) k_rk4_brick(HalfArgs h)
+{
+    rk4_brick_body<FIRST, PAIR>(h, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // One launch over several independent batches (problems of different sizes, steps and
@@ -1632,6 +1810,12 @@ void fill_coefs(void* dst, double nu, double cx, double cy, double cz, double dx
 
 namespace {
 
+// The split variant's brick shape (its k chunk is the brick's).
+bool is_brick(const FusedTile& t)
+{
+    return t.variant == SP_KERNEL_SPLIT && t.tx == BrickCfg::BX && t.ty == BrickCfg::BY && t.nt == BrickCfg::NT;
+}
+
 int fill_args(FusedArgs& a, const FusedStep& st, const FusedTile& tile, View in, View out, int isz, int osz)
 {
     a.in = in;
@@ -1646,7 +1830,7 @@ int fill_args(FusedArgs& a, const FusedStep& st, const FusedTile& tile, View in,
     a.ni = st.ni;
     a.nj = st.nj;
     a.nk = st.nk;
-    a.kchunk = tile.kchunk > 0 ? min(tile.kchunk, st.nk) : st.nk;
+    a.kchunk = is_brick(tile) ? BrickCfg::BZ : tile.kchunk > 0 ? min(tile.kchunk, st.nk) : st.nk;
     a.tiles_x = (st.ni + tile.tx - 1) / tile.tx;
     const int tiles_y = (st.nj + tile.ty - 1) / tile.ty;
     a.tiles = a.tiles_x * tiles_y;
@@ -1711,6 +1895,15 @@ int launch_quad(hipStream_t s, const FusedStep& st, const FusedTile& tile, View 
     return SP_OK;
 }
 
+// Pair access (two elements per lane) needs even x extent, even strides and origins aligned
+// to two elements of each field's storage type (FP64: 16 bytes).
+bool pair_ok(const FusedStep& st, View in, View out, int isz = 8, int osz = 8)
+{
+    const auto even = [](long long v) { return (v & 1) == 0; };
+    return even(st.ni) && even(in.sj) && even(in.sk) && even(out.sj) && even(out.sk) && even(in.slice) &&
+           even(out.slice) && ((uintptr_t)in.p % (2 * isz)) == 0 && ((uintptr_t)out.p % (2 * osz)) == 0;
+}
+
 // Launch A (in -> work: v2) and launch B (work, in -> out: q').  Requires st.work.
 int launch_split(hipStream_t s, const FusedStep& st, const FusedTile& tile, View in, View out)
 {
@@ -1729,6 +1922,18 @@ int launch_split(hipStream_t s, const FusedStep& st, const FusedTile& tile, View
     B.q = in;
     B.q_bytes = A.a.in_bytes;
     const dim3 grid(nblocks_of(A.a, st.nslices));
+    if (is_brick(tile)) {
+        // each launch by its own fields' alignment (the work field's rows are ni long)
+        const bool even = (st.ni & 1) == 0;
+        if (even && pair_ok(st, in, wv)) hipLaunchKernelGGL((k_rk4_brick<true, true>), grid, dim3(BrickCfg::NT), 0, s, A);
+        else hipLaunchKernelGGL((k_rk4_brick<true, false>), grid, dim3(BrickCfg::NT), 0, s, A);
+        SP_HIP(hipGetLastError());
+        if (even && pair_ok(st, in, wv) && pair_ok(st, wv, out))
+            hipLaunchKernelGGL((k_rk4_brick<false, true>), grid, dim3(BrickCfg::NT), 0, s, B);
+        else hipLaunchKernelGGL((k_rk4_brick<false, false>), grid, dim3(BrickCfg::NT), 0, s, B);
+        SP_HIP(hipGetLastError());
+        return SP_OK;
+    }
 #define SP_SPLIT_CASE(TX_, TY_, NT_)                                                           \
     if (tile.tx == TX_ && tile.ty == TY_ && tile.nt == NT_) {                                  \
         hipLaunchKernelGGL((k_rk4_half_pair<TX_, TY_, NT_, true>), grid, dim3(NT_), 0, s, A);  \
@@ -1743,15 +1948,6 @@ int launch_split(hipStream_t s, const FusedStep& st, const FusedTile& tile, View
     SP_SPLIT_CASE(16, 16, 256)
 #undef SP_SPLIT_CASE
     return fail(SP_ERR_UNSUPPORTED, "fused RK4 (split): unsupported tile shape");
-}
-
-// Pair access (two elements per lane) needs even x extent, even strides and origins aligned
-// to two elements of each field's storage type (FP64: 16 bytes).
-bool pair_ok(const FusedStep& st, View in, View out, int isz = 8, int osz = 8)
-{
-    const auto even = [](long long v) { return (v & 1) == 0; };
-    return even(st.ni) && even(in.sj) && even(in.sk) && even(out.sj) && even(out.sk) && even(in.slice) &&
-           even(out.slice) && ((uintptr_t)in.p % (2 * isz)) == 0 && ((uintptr_t)out.p % (2 * osz)) == 0;
 }
 
 template <typename SI, typename SO, typename T>
@@ -1839,11 +2035,13 @@ int launch_rk4_grouped(hipStream_t s, const FusedTile& tile, int in_dtype, int o
     return fail(SP_ERR_UNSUPPORTED, "grouped fused RK4: unsupported dtype pair");
 }
 
+bool fused_tile_brick(const FusedTile& t) { return is_brick(t); }
+
 bool fused_tile_supported(const FusedTile& t, int /*compute_f64*/)
 {
     static const int scalar[][3] = {{32, 32, 1024}, {32, 24, 1024}, {24, 24, 1024}, {32, 16, 512}, {16, 16, 256}};
     static const int pair[][3] = {{32, 32, 512}, {32, 16, 512}, {16, 16, 256}};
-    static const int split[][3] = {{32, 32, 512}, {32, 16, 512}, {32, 16, 256}, {16, 16, 256}};
+    static const int split[][3] = {{32, 32, 512}, {32, 16, 512}, {32, 16, 256}, {16, 16, 256}, {16, 16, 384}};
     if (t.variant == SP_KERNEL_QUAD) return t.tx == QuadCfg::TX && t.ty == QuadCfg::TY && t.nt == QuadCfg::NT;
     if (t.variant == SP_KERNEL_SPLIT) {
         for (const auto& sh : split)
@@ -1860,20 +2058,64 @@ bool fused_tile_supported(const FusedTile& t, int /*compute_f64*/)
     return false;
 }
 
-FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64)
+namespace {
+
+long long tiles_of(int ni, int nj, int nslices, int tx, int ty)
 {
-    // Measured on MI355X (FP64; 16 x 128^3, 8 x 160^3, 24 x 96^3, 1 x 128^3): the 2x2
-    // kernel (32x32 tiles of 512 threads) is fastest once the tiles alone give one block
-    // per CU; below that, x-pair 32x16 tiles chunked in k fill the chip better.  FP32 / BF16
-    // storage runs the x-pair kernel in the 2x2 kernel's place (16 x 128^3: 218 us against
-    // 283 us for the scalar kernel's best tile; 1 x 384^3 in 64-plane chunks: 479 against
+    return (long long)((ni + tx - 1) / tx) * ((nj + ty - 1) / ty) * nslices;
+}
+
+// The k chunk of 32x32 tiles for which the blocks finish first, and that time in planes: one
+// block per CU runs at a time, each walks its chunk and `fill` planes more, in groups of `group`.
+int best_kchunk(long long tiles, int nk, int fill, int group, double* planes)
+{
+    int best = nk;
+    *planes = 1e30;
+    for (int chunks = 1; chunks <= nk / 8 || chunks == 1; ++chunks) {
+        const int kc = (nk + chunks - 1) / chunks;
+        const long long blocks = tiles * ((nk + kc - 1) / kc);
+        const double t = (double)((blocks + 255) / 256) * ((kc + fill + group - 1) / group * group);
+        if (t < *planes) {
+            *planes = t;
+            best = kc;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, bool one_launch)
+{
+    // FP64: the 2x2 kernel with the k chunk that finishes first, or bricks (two launches) while
+    // those are few.  Measured on MI355X in us per step:
+    //   2x2: 1.25-1.4 per plane and round of 256 blocks (1 x 256^3 in 64-plane chunks 120, 4 x
+    //   128^3 in 32-plane chunks 73, 16 x 128^3 210, 1 x 384^3 in 128-plane chunks 389); the
+    //   whole-k and 64-plane chunks chosen before: 1 x 256^3 250, 4 x 128^3 155, 1 x 384^3 437.
+    //   bricks: 14 up to 256 of them, then 8 + 0.033 each (1 x 64^3 14.1 against 35 for the 2x2
+    //   kernel; 432 bricks, 1 x 96^3: 23 against 35; 1024, 1 x 128^3: 41 against 36).
+    // Odd x extents cannot take the 2x2 kernel's 16-byte accesses: bricks (0.055 each; 1024
+    // bricks, 127^3: 56) or the scalar kernel (127^3 56, 161^3 148 in 64-plane chunks against 145 for
+    // bricks, 255^3 287 against 441).
+    const long long bricks = tiles_of(ni, nj, nslices, 16, 16) * ((nk + 7) / 8);
+    if (compute_f64 && !one_launch) {
+        const FusedTile brick{16, 16, 384, 8, SP_KERNEL_SPLIT};
+        if (ni & 1) {
+            if (bricks <= 2048) return brick;
+        } else {
+            double planes;
+            const int kc = best_kchunk(tiles_of(ni, nj, nslices, 32, 32), nk, 18, 4, &planes);
+            if (std::max(14., 8. + 0.033 * bricks) < 1.3 * planes) return brick;
+            return FusedTile{32, 32, 512, kc >= nk ? 0 : kc, SP_KERNEL_QUAD};
+        }
+    }
+    // One launch per step only, reduced-precision storage, and odd extents past the bricks.
+    // FP32 / BF16 storage runs the x-pair kernel in the 2x2 kernel's place (16 x 128^3: 218 us
+    // against 283 us for the scalar kernel's best tile; 1 x 384^3 in 64-plane chunks: 479 against
     // 574 us).  Odd x extents fall back to the scalar kernel at launch.
     const long long want = 256;  // one block per CU
     FusedTile t{32, 32, 512, 0, compute_f64 ? SP_KERNEL_QUAD : SP_KERNEL_PAIR};
-    long long blocks = (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty) * nslices;
-    // Long k columns (one 384^3 slice: 144 tiles): 64-plane chunks of 32x32 tiles give three
-    // or more blocks per CU at a 19-plane pipeline fill (measured, FP64: 0.55 ms per 384^3
-    // step, against 1.07 ms for whole-k 32x16 tiles, whose 288 blocks leave a ragged second wave).
+    long long blocks = tiles_of(ni, nj, nslices, t.tx, t.ty);
     if (blocks < want && blocks * (nk / 64) >= 3 * want) {
         t.kchunk = 64;
         return t;
@@ -1881,7 +2123,7 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64)
     if (blocks < want) {
         t.ty = 16;
         t.variant = SP_KERNEL_PAIR;
-        blocks = (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty) * nslices;
+        blocks = tiles_of(ni, nj, nslices, t.tx, t.ty);
     }
     int chunks = (int)((want + blocks - 1) / blocks);
     if (chunks < 1) chunks = 1;
@@ -1895,7 +2137,7 @@ void fused_candidates(int ni, int nj, int nk, int nslices, int compute_f64, std:
 {
     static const int scalar[][3] = {{32, 32, 1024}, {32, 24, 1024}, {24, 24, 1024}, {32, 16, 512}, {16, 16, 256}};
     static const int pair[][3] = {{32, 32, 512}, {32, 16, 512}, {16, 16, 256}};
-    static const int split[][3] = {{32, 32, 512}, {32, 16, 512}, {32, 16, 256}, {16, 16, 256}};
+    static const int split[][3] = {{32, 32, 512}, {32, 16, 512}, {32, 16, 256}, {16, 16, 256}, {16, 16, 384}};
     std::vector<FusedTile> shapes;
     if (!compute_f64 && ni % 2 == 0)
         for (const auto& sh : pair) shapes.push_back(FusedTile{sh[0], sh[1], sh[2], 0, SP_KERNEL_PAIR});
@@ -1906,18 +2148,26 @@ void fused_candidates(int ni, int nj, int nk, int nslices, int compute_f64, std:
         // within 64 MiB (the last-level cache holds the three)
         if (split_work_bytes(ni, nj, nk, nslices) <= (64u << 20))
             for (const auto& sh : split) shapes.push_back(FusedTile{sh[0], sh[1], sh[2], 0, SP_KERNEL_SPLIT});
-    }
+    } else if (compute_f64 && split_work_bytes(ni, nj, nk, nslices) <= (64u << 20))
+        shapes.push_back(FusedTile{BrickCfg::BX, BrickCfg::BY, BrickCfg::NT, 0, SP_KERNEL_SPLIT});
     for (const auto& sh : scalar) shapes.push_back(FusedTile{sh[0], sh[1], sh[2], 0, SP_KERNEL_SCALAR});
     out.clear();
     for (const FusedTile& t : shapes) {
-        const long long blocks = (long long)((ni + t.tx - 1) / t.tx) * ((nj + t.ty - 1) / t.ty) * nslices;
-        // k chunks: the whole extent, and shorter ones (>= 16 planes, >= 8 for the split
-        // kernel's 9-plane fill) only while the tiles alone give fewer than 4 blocks per CU
-        const int cmin = t.variant == SP_KERNEL_SPLIT ? 8 : 16;
+        if (is_brick(t)) {
+            out.push_back(FusedTile{t.tx, t.ty, t.nt, BrickCfg::BZ, t.variant});
+            continue;
+        }
+        const long long blocks = tiles_of(ni, nj, nslices, t.tx, t.ty);
+        // k chunks: the whole extent, and shorter ones (>= 16 planes, >= 8 for the 2x2 and split
+        // kernels) only while the tiles alone give fewer than 4 blocks per CU
+        const int cmin = t.variant == SP_KERNEL_SPLIT || t.variant == SP_KERNEL_QUAD ? 8 : 16;
         std::vector<int> kcs{0};
+        double planes;
+        const int best = t.variant == SP_KERNEL_QUAD ? best_kchunk(blocks, nk, 18, 4, &planes) : 0;
         if (blocks < 1024)
             for (int c : {nk / 2, nk / 4, nk / 8, 64, 32, 16, 8})
                 if (c >= cmin && c < nk && std::find(kcs.begin(), kcs.end(), c) == kcs.end()) kcs.push_back(c);
+        if (best > 0 && best < nk && std::find(kcs.begin(), kcs.end(), best) == kcs.end()) kcs.push_back(best);
         for (int c : kcs) {
             FusedTile x = t;
             x.kchunk = c;
@@ -1944,7 +2194,8 @@ int launch_rk4_fused(hipStream_t s, const FusedStep& st, const FusedTile& tile_i
         if (in_dtype == SP_F64 && out_dtype == SP_BF16) return launch_pair<double, bf16, float>(s, st, tile, in, out);
         if (in_dtype == SP_BF16 && out_dtype == SP_BF16) return launch_pair<bf16, bf16, float>(s, st, tile, in, out);
     }
-    if (f64 && tile.variant == SP_KERNEL_SPLIT && pair_ok(st, in, out)) return launch_split(s, st, tile, in, out);
+    if (f64 && tile.variant == SP_KERNEL_SPLIT && (is_brick(tile) || pair_ok(st, in, out)))
+        return launch_split(s, st, tile, in, out);
     if (tile.variant == SP_KERNEL_PAIR || tile.variant == SP_KERNEL_QUAD || tile.variant == SP_KERNEL_SPLIT) {
         // odd sizes, unaligned views or reduced-precision storage: the scalar kernel with
         // its fastest FP64 shape and the caller's k chunk

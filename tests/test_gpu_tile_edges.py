@@ -44,3 +44,13 @@ def test_quad_kernel_edges(sp, shape, kchunk):
     assert np.array_equal(got, ref)
     exact = O.OConvection(*shape, 1. / 32, 0.02, 0.0, *C3).rk4(q0, 0.0, 1e-4, 3)
     assert np.abs(got - exact).max() <= 1e-12 * np.abs(exact).max()
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 8), (3, 5, 8), (8, 8, 8), (16, 16, 16), (17, 16, 9), (18, 33, 15), (31, 7, 24), (48, 34, 33)],
+                         ids=lambda s: "%dx%dx%d" % s)
+def test_brick_kernel_edges(sp, shape):
+    q0, ref = run(sp, shape, "scalar", (32, 16, 512), 0, steps=4, nufreq=30.0)
+    _, got = run(sp, shape, "split", (16, 16, 384), 8, steps=4, nufreq=30.0)
+    assert np.array_equal(got, ref)
+    exact = O.OConvection(*shape, 1. / 32, 0.02, 30.0, *C3).rk4(q0, 0.0, 1e-4, 4)
+    assert np.abs(got - exact).max() <= 1e-12 * np.abs(exact).max()
