@@ -26,7 +26,7 @@ using namespace sp;
 
 namespace {
 
-constexpr int kCorrBlocks = 64;  // blocks (and partial sums) per slice correction
+constexpr int kCorrBlocks = 128;  // blocks (and partial sums) per slice correction
 
 struct Prob {
     sp_problem d{};
