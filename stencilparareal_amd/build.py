@@ -34,7 +34,7 @@ SOURCES = {
     "sp_batch.hip": [],
     "sp_spectral.hip": [],
 }
-HEADERS = ["sp_internal.hpp", "sp_handles.hpp", os.path.join("..", "..", "include", "stencilparareal.h")]
+HEADERS = ["sp_device.hpp", "sp_internal.hpp", "sp_handles.hpp", os.path.join("..", "..", "include", "stencilparareal.h")]
 
 
 def hipcc() -> str:

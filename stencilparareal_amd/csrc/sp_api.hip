@@ -345,24 +345,46 @@ int rk4_staged_step(sp_prop* p, View vin, View vout, double t, double dt)
     return SP_OK;
 }
 
-// Forward Euler steps (DoEuler), f64, with ping-pong so the fused sweep never runs in place.
+// Euler steps as launches of two where the fields allow it, then of one.
+struct EulerLaunches {
+    int two, one;
+    int count() const { return two + one; }
+};
+EulerLaunches euler_launches(const StagedParams& P, View in, View out, View scratch, int steps)
+{
+    const int two = euler_two_steps(P, in, out) && euler_two_steps(P, scratch, scratch) ? steps / 2 : 0;
+    return {two, steps - 2 * two};
+}
+// Launch l of them, with nu of the propagator's step i from nu_of(i).
+template <typename F>
+int euler_launch(hipStream_t s, const StagedParams& P, const EulerLaunches& n, int l, View src, View dst, F nu_of,
+                 double dt, int upwind, int nslices)
+{
+    if (l >= n.two) return launch_euler_fused(s, P, src, dst, nu_of(n.two + l), dt, upwind, nslices);
+    const double nu[2] = {nu_of(2 * l), nu_of(2 * l + 1)};
+    return launch_euler_two(s, P, src, dst, nu, dt, upwind, nslices);
+}
+
+// Forward Euler steps (DoEuler), f64, with ping-pong so no launch runs in place.
 int euler_run(sp_prop* p, View vin, View vout, bool aliased, double t0, double dt, int steps, int nslices,
               View scrA, View scrB)
 {
     hipStream_t s = p->ctx->stream;
     const StagedParams P{p->ni, p->nj, p->nk, p->cx, p->cy, p->cz, p->dx, p->dx * p->dx};
+    const EulerLaunches n = euler_launches(P, vin, vout, scrA, steps);
+    const int launches = n.count();
     View src = vin;
-    for (int i = 0; i < steps; ++i) {
-        const int left = steps - 1 - i;
+    for (int l = 0; l < launches; ++l) {
+        const int left = launches - 1 - l;
         View dst;
         if (!aliased) dst = (left % 2 == 0) ? vout : scrA;
-        else if (left == 0 && steps > 1) dst = vout;
-        else dst = (i % 2 == 0) ? scrA : scrB;
-        const double nu = computenu(p, t0 + i * dt);
-        SP_TRY(launch_euler_fused(s, P, src, dst, nu, dt, p->upwind, nslices));
+        else if (left == 0 && launches > 1) dst = vout;
+        else dst = (l % 2 == 0) ? scrA : scrB;
+        SP_TRY(euler_launch(s, P, n, l, src, dst, [&](int i) { return computenu(p, t0 + i * dt); }, dt, p->upwind,
+                            nslices));
         src = dst;
     }
-    if (aliased && steps == 1) SP_TRY(launch_convert(s, p->ni, p->nj, p->nk, nslices, SP_F64, scrA, SP_F64, vout));
+    if (aliased && launches == 1) SP_TRY(launch_convert(s, p->ni, p->nj, p->nk, nslices, SP_F64, scrA, SP_F64, vout));
     return SP_OK;
 }
 
@@ -987,31 +1009,34 @@ int coarse_run(sp_parareal* pr, int nslices, int slice0, int idt, View src, View
         }
         return SP_OK;
     }
+    // nu of sub-step i (one slice, or all slices at the same time)
+    const auto nu_of = [&](int i) {
+        if (first_index >= 0) return computenu(p, 0. + (double)(first_index + i) * pr->dtG);
+        if (pr->nu_const || nslices > 1) return p->nu0;
+        return pr->nuG_host[(size_t)i * pr->S + slice0];
+    };
     View cur = src;
     int cdt = idt;
+    if (pr->cfg.coarse_kind != SP_COARSE_RK4) {
+        if (first_index < 0 && !pr->nu_const && nslices > 1)
+            return fail(SP_ERR_UNSUPPORTED, "batched Euler coarse with time-dependent nu");
+        const StagedParams P{p->ni, p->nj, p->nk, p->cx, p->cy, p->cz, p->dx, p->dx * p->dx};
+        const EulerLaunches n = euler_launches(P, src, dst, scr, steps);
+        for (int l = 0; l < n.count(); ++l) {
+            const View d = ((n.count() - 1 - l) % 2 == 0) ? dst : scr;
+            SP_TRY(euler_launch(s, P, n, l, cur, d, nu_of, pr->dtG, p->upwind, nslices));
+            cur = d;
+        }
+        return SP_OK;
+    }
     for (int i = 0; i < steps; ++i) {
         const int left = steps - 1 - i;
         const View d = (left % 2 == 0) ? dst : scr;
-        double nu;
         const void* nud = nullptr;
-        if (first_index >= 0) {
-            nu = computenu(p, 0. + (double)(first_index + i) * pr->dtG);
-        } else if (pr->nu_const) {
-            nu = p->nu0;
-        } else if (nslices == 1) {
-            nu = pr->nuG_host[(size_t)i * pr->S + slice0];
-        } else {
-            nu = p->nu0;
+        if (first_index < 0 && !pr->nu_const && nslices > 1)
             nud = (const char*)coef_base + ((size_t)i * pr->S + slice0) * coefs_size();
-        }
-        if (pr->cfg.coarse_kind == SP_COARSE_RK4) {
-            const FusedTile& tile = gdt != pr->gdt ? pr->tileG1_64 : nslices == 1 ? pr->tileG1 : pr->tileGS;
-            SP_TRY(launch_rk4_fused(s, pr_step(pr, nslices, pr->dtG, nud, nu), tile, cdt, cur, gdt, d));
-        } else {
-            if (nud) return fail(SP_ERR_UNSUPPORTED, "batched Euler coarse with time-dependent nu");
-            const StagedParams P{p->ni, p->nj, p->nk, p->cx, p->cy, p->cz, p->dx, p->dx * p->dx};
-            SP_TRY(launch_euler_fused(s, P, cur, d, nu, pr->dtG, p->upwind, nslices));
-        }
+        const FusedTile& tile = gdt != pr->gdt ? pr->tileG1_64 : nslices == 1 ? pr->tileG1 : pr->tileGS;
+        SP_TRY(launch_rk4_fused(s, pr_step(pr, nslices, pr->dtG, nud, nu_of(i)), tile, cdt, cur, gdt, d));
         cur = d;
         cdt = gdt;
     }

@@ -39,6 +39,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "sp_device.hpp"
 #include "sp_internal.hpp"
 
 namespace sp {
@@ -95,26 +96,6 @@ __device__ __forceinline__ StarW<float> load_w<float>(const Coefs& k)
                         k.wf[9], k.wf[10], k.wf[11], k.wf[12], k.ff[0], k.ff[1], k.ff[2], k.ff[3]};
 }
 
-__device__ __forceinline__ int pmod(int a, int n)
-{
-    int r = a % n;
-    return r < 0 ? r + n : r;
-}
-
-// Plane index p in [-3n, 4n) wrapped into [0, n) without branches (scalar selects).  The
-// stream touches planes z0-18 .. zend+16, inside that range for n >= 8; the host sends
-// smaller k extents to the reference-order path.
-__device__ __forceinline__ int wrapz(int p, int n)
-{
-    p += p < 0 ? n : 0;
-    p += p < 0 ? n : 0;
-    p += p < 0 ? n : 0;
-    p -= p >= n ? n : 0;
-    p -= p >= n ? n : 0;
-    p -= p >= n ? n : 0;
-    return p;
-}
-
 // Stage geometry: stage s (1..4) computes a (TX+2h) x (TY+2h) region, h = 8-2s, from an
 // input plane of (TX+2h+4) x (TY+2h+4) held in LDS.
 template <int TX, int TY, int S>
@@ -161,16 +142,6 @@ __device__ __forceinline__ void stage_step(const T* __restrict__ P, const StarW<
         // small enough for 16 waves per CU; the other waves hide the LDS latency
         __builtin_amdgcn_sched_barrier(0);
     }
-}
-
-// Buffer-resource access: one SGPR descriptor per field, 32-bit per-lane byte offsets
-// and the plane offset in an SGPR, so the k stream needs no 64-bit address arithmetic.
-// Out-of-range offsets read 0 / drop the store instead of faulting.
-#define SP_RSRC_DWORD3 0x00020000  // gfx9 family raw buffer (as composable_kernel uses)
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, unsigned bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, SP_RSRC_DWORD3);
 }
 
 template <typename S>
@@ -237,15 +208,6 @@ __device__ __forceinline__ void stage_qload(T (&qv)[M], __amdgpu_buffer_rsrc_t r
 {
 #pragma unroll
     for (int m = 0; m < M; ++m) qv[m] = (T)Buf<SI>::ld(r, cl.q[m], zo);
-}
-
-// Blocks are handed to the 8 XCDs round-robin (block b runs on XCD b % 8).  Renumber so
-// that each XCD receives a contiguous range of tiles: neighbouring tiles, which read each
-// other's halo columns, then share one L2.  (The first n % 8 XCDs get one block more.)
-__device__ __forceinline__ int xcd_block(int b, int n)
-{
-    const int x = b % 8, r = n % 8;
-    return x * (n / 8) + min(x, r) + b / 8;
 }
 
 template <typename SI, typename SO, typename T, int TX, int TY, int NT>
@@ -442,13 +404,6 @@ __device__ __forceinline__ void st2_stream(__amdgpu_buffer_rsrc_t r, int vo, int
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, vo, so, 2);
 }
-// 16 bytes per lane from global memory straight into LDS: lane l of the wave writes
-// lds + 16 l (lds: the wave's base, the same for every lane).
-__device__ __forceinline__ void ld2_to_lds(__amdgpu_buffer_rsrc_t r, double* lds, int vo, int so)
-{
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, vo, so, 0, 0);
-}
-
 // Two x-adjacent values of compute type T (d2 for FP64), and their global access for
 // storage type S: 2 * sizeof(S) bytes per lane (FP64 16, FP32 8, BF16 4), converted to T.
 template <typename T>
@@ -1238,24 +1193,6 @@ __device__ __forceinline__ void quad_zero(double (&acc)[N][4])
     for (int j = 0; j < N; ++j) acc[j][0] = acc[j][1] = acc[j][2] = acc[j][3] = 0.;
 }
 
-// Waits until at most N of this wave's vector-memory accesses are outstanding (they complete
-// in the order of issue).
-template <int N>
-__device__ __forceinline__ void vm_wait() { __builtin_amdgcn_s_waitcnt(0x0F70 | N); }
-
-// Workgroup barrier for LDS data: this wave's LDS accesses are complete before it, but for the
-// last N issued (reads of planes that nobody writes next), and none moves across it.  Unlike __syncthreads it leaves loads into LDS in flight (vm_wait before it
-// for those that another wave reads next).
-template <int N = 0>
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_s_waitcnt(0xC07F | N << 8);  // lgkmcnt(N)
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 __device__ __forceinline__ void rk4_quad_body(const FusedArgs& a, const int bid)
 {
     using Q = QuadCfg;
@@ -1632,34 +1569,7 @@ __device__ __forceinline__ void rk4_brick_body(const HalfArgs& h, const int bid)
     const int iskb = (int)a.in.sk * 8, qskb = (int)h.q.sk * 8, oskb = (int)a.out.sk * 8;
     const StarW<double> w = a.cdev ? load_w<double>(a.cdev[slice]) : load_w<double>(a.c);
 
-    // The input's planes, each 312 16-byte slots in the order of the cells: waves 0-4 load a
-    // slot per lane, or (not PAIR) four words per lane.
-    if (wave < 5) {
-        constexpr int M = PAIR ? 1 : 4;
-        int off[M];
-        bool in[M];
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const int e = PAIR ? 2 * (wave * 64 + lane) : wave * 128 + m * 32 + (lane >> 1);  // cell of the plane
-            in[m] = e < B::PLANE;
-            off[m] = (pmod(x0 - 4 + e % B::W, ni) + pmod(y0 - 4 + e / B::W, nj) * (int)a.in.sj) * 8 +
-                     (PAIR ? 0 : (lane & 1) * 4);
-        }
-#pragma unroll
-        for (int p = 0; p < B::D; ++p) {
-            const int zo = wrapz(z0 - 4 + p, nk) * iskb;
-#pragma unroll
-            for (int m = 0; m < M; ++m) {
-                double* const dst = P + p * B::PLANE + wave * 128 + m * 32;
-                if (in[m]) {
-                    if constexpr (PAIR) ld2_to_lds(rin, dst, off[m], zo);
-                    else
-                        __builtin_amdgcn_raw_ptr_buffer_load_lds(rin, (__attribute__((address_space(3))) void*)dst, 4,
-                                                                 off[m], zo, 0, 0);
-                }
-            }
-        }
-    }
+    brick_load<PAIR, B::W, B::H, B::D>(P, rin, iskb, (int)a.in.sj, x0 - 4, y0 - 4, z0 - 4, ni, nj, nk, wave, lane);
     // first stage: column 96 zg + s of three planes; s in rows of 8, 10 (eight times), 8 blocks
     const int za = tid / 96, sa = tid % 96;
     const int by = sa < 8 ? -1 : sa < 88 ? (sa - 8) / 10 : 8;

@@ -133,6 +133,12 @@ int launch_rk_stage(hipStream_t s, const StagedParams& P, View qin, View k1, Vie
 int launch_euler_fused(hipStream_t s, const StagedParams& P, View qin, View qout, double nu, double dt,
                        int upwind, int nslices);
 
+// Two such steps in one launch, nu[i] step i's (several slices: all at the same nu), for fields
+// that euler_two_steps accepts.
+bool euler_two_steps(const StagedParams& P, View qin, View qout);
+int launch_euler_two(hipStream_t s, const StagedParams& P, View qin, View qout, const double nu[2], double dt, int upwind,
+                     int nslices);
+
 // Fused RK4 step over `nslices` batched slices.  Types by dtype codes.
 struct FusedTile {
     int tx, ty, nt, kchunk;
