@@ -1975,18 +1975,26 @@ long long tiles_of(int ni, int nj, int nslices, int tx, int ty)
     return (long long)((ni + tx - 1) / tx) * ((nj + ty - 1) / ty) * nslices;
 }
 
-// The k chunk of 32x32 tiles for which the blocks finish first, and that time in planes: one
-// block per CU runs at a time, each walks its chunk and `fill` planes more, in groups of `group`.
-int best_kchunk(long long tiles, int nk, int fill, int group, double* planes)
+// A streaming kernel's time in us: each block walks its k chunk and `fill` planes more, in groups
+// of `group`.  A plane of a round of 256 blocks (one per CU) takes `first`, and `more` for every
+// round where several blocks share a CU.
+struct WalkCost {
+    int fill, group;
+    double first, more;
+};
+constexpr WalkCost kQuadWalk{18, 4, 1.3, 1.3};
+
+// The k chunk for which the blocks of these tiles finish first, and that time.
+int best_kchunk(long long tiles, int nk, const WalkCost& c, double* us)
 {
     int best = nk;
-    *planes = 1e30;
+    *us = 1e30;
     for (int chunks = 1; chunks <= nk / 8 || chunks == 1; ++chunks) {
         const int kc = (nk + chunks - 1) / chunks;
-        const long long blocks = tiles * ((nk + kc - 1) / kc);
-        const double t = (double)((blocks + 255) / 256) * ((kc + fill + group - 1) / group * group);
-        if (t < *planes) {
-            *planes = t;
+        const long long rounds = (tiles * ((nk + kc - 1) / kc) + 255) / 256;
+        const double t = std::max(c.first, c.more * rounds) * ((kc + c.fill + c.group - 1) / c.group * c.group);
+        if (t < *us) {
+            *us = t;
             best = kc;
         }
     }
@@ -2013,16 +2021,35 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
         if (ni & 1) {
             if (bricks <= 2048) return brick;
         } else {
-            double planes;
-            const int kc = best_kchunk(tiles_of(ni, nj, nslices, 32, 32), nk, 18, 4, &planes);
-            if (std::max(14., 8. + 0.033 * bricks) < 1.3 * planes) return brick;
+            double us;
+            const int kc = best_kchunk(tiles_of(ni, nj, nslices, 32, 32), nk, kQuadWalk, &us);
+            if (std::max(14., 8. + 0.033 * bricks) < us) return brick;
             return FusedTile{32, 32, 512, kc >= nk ? 0 : kc, SP_KERNEL_QUAD};
         }
     }
-    // One launch per step only, reduced-precision storage, and odd extents past the bricks.
-    // FP32 / BF16 storage runs the x-pair kernel in the 2x2 kernel's place (16 x 128^3: 218 us
-    // against 283 us for the scalar kernel's best tile; 1 x 384^3 in 64-plane chunks: 479 against
-    // 574 us).  Odd x extents fall back to the scalar kernel at launch.
+    // FP32 / BF16 storage: the x-pair kernel in the tile and k chunk that finish first.  Measured in
+    // FP32, us per plane (BF16 5-20 % more): 32x32 1.46 per round, 32x16 1.05 alone and 0.78 per
+    // round of two and more, 16x16 0.88 and 0.60.  1 x 64^3 16x16 in 8-plane chunks 23.6 us (34.5
+    // for 32x16 in 16), 1 x 256^3 32x32 in 64 122 (154 for 32x16 in 128), 1 x 384^3 32x32 in 77-80
+    // 435 (479 in 64; BF16 526 against 598, its best, 32x16 in 64, 499).
+    if (!compute_f64 && !one_launch && !(ni & 1)) {
+        static constexpr struct {
+            int tx, ty, nt;
+            WalkCost cost;
+        } shapes[] = {{32, 32, 512, {19, 1, 1.46, 1.46}},
+                      {32, 16, 512, {19, 1, 1.05, 0.78}},
+                      {16, 16, 256, {19, 1, 0.88, 0.60}}};
+        FusedTile t{};
+        double least = 1e30;
+        for (const auto& sh : shapes) {
+            double us;
+            const int kc = best_kchunk(tiles_of(ni, nj, nslices, sh.tx, sh.ty), nk, sh.cost, &us);
+            if (us < least) t = FusedTile{sh.tx, sh.ty, sh.nt, kc >= nk ? 0 : kc, SP_KERNEL_PAIR}, least = us;
+        }
+        return t;
+    }
+    // One launch per step (which other problems may share), and odd extents past the bricks: the
+    // scalar kernel in reduced precision and where accesses are not aligned.
     const long long want = 256;  // one block per CU
     FusedTile t{32, 32, 512, 0, compute_f64 ? SP_KERNEL_QUAD : SP_KERNEL_PAIR};
     long long blocks = tiles_of(ni, nj, nslices, t.tx, t.ty);
@@ -2072,8 +2099,8 @@ void fused_candidates(int ni, int nj, int nk, int nslices, int compute_f64, std:
         // kernels) only while the tiles alone give fewer than 4 blocks per CU
         const int cmin = t.variant == SP_KERNEL_SPLIT || t.variant == SP_KERNEL_QUAD ? 8 : 16;
         std::vector<int> kcs{0};
-        double planes;
-        const int best = t.variant == SP_KERNEL_QUAD ? best_kchunk(blocks, nk, 18, 4, &planes) : 0;
+        double us;
+        const int best = t.variant == SP_KERNEL_QUAD ? best_kchunk(blocks, nk, kQuadWalk, &us) : 0;
         if (blocks < 1024)
             for (int c : {nk / 2, nk / 4, nk / 8, 64, 32, 16, 8})
                 if (c >= cmin && c < nk && std::find(kcs.begin(), kcs.end(), c) == kcs.end()) kcs.push_back(c);
