@@ -13,6 +13,14 @@ __device__ __forceinline__ int pmod(int a, int n)
     return r < 0 ? r + n : r;
 }
 
+// a in [-n, 2n) where n >= 24 (block-uniform), any a otherwise: two selects instead of a division
+__device__ __forceinline__ int near_mod(int a, int n)
+{
+    if (n < 24) return pmod(a, n);
+    a += a < 0 ? n : 0;
+    return a - (a >= n ? n : 0);
+}
+
 // Plane index p in [-3n, 4n) wrapped into [0, n) without branches (scalar selects).  The
 // stream touches planes z0-18 .. zend+16, inside that range for n >= 8; the host sends
 // smaller k extents to the reference-order path.
@@ -76,7 +84,7 @@ __device__ __forceinline__ void lds_barrier()
 }
 
 // Loads a brick of D planes of H rows of W doubles (W even, at most 640 cells per plane) from
-// (x, y, z) on, with periodic images, into P in the order of its cells, straight into LDS: a
+// (x, y, z) on (x and y at most 24 cells outside the field), with periodic images, into P in the order of its cells, straight into LDS: a
 // plane's 16-byte slots by the lanes of waves 0 to 4, or (not PAIR: rows that are not 16-byte
 // aligned pairs) four words per lane.  The caller waits for the loads (vm_wait, barrier).
 template <bool PAIR, int W, int H, int D>
@@ -92,7 +100,7 @@ __device__ __forceinline__ void brick_load(double* P, __amdgpu_buffer_rsrc_t r, 
     for (int m = 0; m < M; ++m) {
         const int e = PAIR ? 2 * (wave * 64 + lane) : wave * 128 + m * 32 + (lane >> 1);  // cell of the plane
         in[m] = e < W * H;
-        off[m] = (pmod(x + e % W, ni) + pmod(y + e / W, nj) * sj) * 8 + (PAIR ? 0 : (lane & 1) * 4);
+        off[m] = (near_mod(x + e % W, ni) + near_mod(y + e / W, nj) * sj) * 8 + (PAIR ? 0 : (lane & 1) * 4);
     }
 #pragma unroll
     for (int p = 0; p < D; ++p) {

@@ -825,6 +825,8 @@ struct HalfArgs {
     FusedArgs a;       // a.in: u; a.out: the output
     View q;            // the update base (launch A: the same field as a.in)
     unsigned q_bytes;  // bytes one slice of q spans from its origin
+    int bricks;        // brick kernel: bricks of all slices, (2^32 - 1) over each divisor
+    unsigned inv_tiles, inv_chunks, inv_tiles_x;
 };
 
 template <int TX, int TY, int NT, bool FIRST>
@@ -1483,19 +1485,25 @@ __device__ __forceinline__ void rk4_quad_body(const FusedArgs& a, const int bid)
 // A small field has too few tiles to fill the chip, and a chunk's walk along k is bound by one
 // plane's latency (0.5-1.2 us) times its planes, most of which fill the pipeline.  Here nothing
 // walks: a block loads the whole input of a 16x16x8 brick of results at once (24x24x16 cells,
-// 80 KB of LDS, two blocks per CU), computes one stage on its 20x20x12 cells (without the
-// corners, 96 2x2 columns x 12 planes over 384 lanes, three planes each), puts the result over
-// the input in LDS and computes the next stage.  Four stages take two launches through the
-// work field of the split step:
+// 74 KB of LDS), computes one stage on the cells that the next one reads (the brick's 64 2x2
+// columns over 12 planes and the 32 columns around it over 8: two planes per lane of eight
+// waves), puts the result over the input in LDS and computes the next stage.  A block takes
+// several bricks in turn where there are more than CUs: two more waves load the next one into a
+// second buffer meanwhile.  Four stages take two launches through the split step's work field:
 //   launch A: u = q,  v_a = q + f1 L u,  out = q + f2 L v_a   (= v2)
 //   launch B: u = v2, v_a = q + f3 L u,  out = q + f4 L v_a   (= q')
 // with the other kernels' operations in the same order (the same bits).  Any sizes, strides and
 // alignment: PAIR loads and stores 16 bytes, otherwise each cell's two words are loaded by
-// lanes of their own.  Conflict-free planes: 10 columns per row of the first stage and a row
-// pair of 26 chunks (10 mod 16) put consecutive lanes on consecutive chunks across rows.
+// lanes of their own.  Eight columns per row and a row pair of 24 chunks of 16 bytes (8 mod 16)
+// put consecutive lanes on consecutive chunks across rows: no bank conflicts.
+// Bound by latency up to 256 bricks (64^3 13.2 us a step), then by memory accesses in flight:
+// 2.9 us per brick and launch, of which loads and stores alone take 2.6 and the stages 1.8.  One
+// brick per block on six waves, loads not overlapped: 64^3 13.9, 128^3 42.0 against 32.5 us, 127^3
+// 52.4 against 40.4, 8 x 64^3 40.3 against 32.1.
 struct BrickCfg {
-    static constexpr int BX = 16, BY = 16, BZ = 8, NT = 384;
-    static constexpr int W = 26, H = 24, D = 16, PLANE = W * H;  // the input's cells in LDS
+    static constexpr int BX = 16, BY = 16, BZ = 8, NT = 384;  // NT: the descriptor's only
+    static constexpr int W = 24, H = 24, D = 16, PLANE = W * H, CELLS = D * PLANE;  // the input's cells in LDS
+    static constexpr int WAVES = 8, THREADS = (WAVES + 2) * 64;                     // the last two load
 };
 
 // The base values q of a lane's 2x2 block in N planes, from global memory.
@@ -1507,12 +1515,18 @@ struct BrickCols {
 #pragma unroll
         for (int f = 0; f < 2; ++f)
 #pragma unroll
-            for (int e = 0; e < (PAIR ? 1 : 2); ++e) o[f][e] = (pmod(x + e, ni) + pmod(y + f, nj) * sj) * 8;
+            for (int e = 0; e < (PAIR ? 1 : 2); ++e) o[f][e] = (near_mod(x + e, ni) + near_mod(y + f, nj) * sj) * 8;
     }
     __device__ __forceinline__ d2 ld(__amdgpu_buffer_rsrc_t r, int f, int zo) const
     {
         if constexpr (PAIR) return ld2(r, o[f][0], zo);
         else return d2{Buf<double>::ld(r, o[f][0], zo), Buf<double>::ld(r, o[f][1], zo)};
+    }
+    // zo of the lane's own
+    __device__ __forceinline__ d2 ld_lane(__amdgpu_buffer_rsrc_t r, int f, int zo) const
+    {
+        if constexpr (PAIR) return ld2(r, o[f][0] + zo, 0);
+        else return d2{Buf<double>::ld(r, o[f][0] + zo, 0), Buf<double>::ld(r, o[f][1] + zo, 0)};
     }
     __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, int f, int zo, d2 v) const
     {
@@ -1549,75 +1563,201 @@ __device__ __forceinline__ void brick_stage(d2 (&v)[N][2], const double* __restr
     }
 }
 
+// A brick's input, with periodic images, straight into LDS in the order of its cells: two planes
+// are nine whole wave loads of 16-byte slots (part 4 is half of each plane) or, where rows are
+// not 16-byte aligned pairs, a plane 18 of single words.  What bounds this is the instructions
+// around a load: masked loads and a general wrap of each plane's index took 50 of them, and 3000
+// cycles for a brick; the byte offset of a plane steps with three.
+template <bool PAIR>
+struct BrickLoads {
+    static constexpr int W = BrickCfg::W, PLANE = BrickCfg::PLANE, N = PAIR ? 9 : 18;
+    static_assert(2 * PLANE / 2 == 9 * 64 && PLANE * 2 == 18 * 64, "whole wave loads");
+    // part t's cell: byte offset in its plane
+    static __device__ __forceinline__ int offset(int t, int lane, int sj, int x, int y, int ni, int nj)
+    {
+        const int e = PAIR ? (2 * (t * 64 + lane)) % PLANE : t * 32 + (lane >> 1);
+        return (near_mod(x + e % W, ni) + near_mod(y + e / W, nj) * sj) * 8 + (PAIR ? 0 : (lane & 1) * 4);
+    }
+    // z, a plane's byte offset below span (all planes'), d < span further on
+    static __device__ __forceinline__ unsigned step(unsigned z, unsigned d, unsigned span)
+    {
+        return min(z + d, z + d - span);  // the second is huge unless the first is past the end
+    }
+    // part t of the plane pair at dst, planes at byte offsets z0 and z1
+    static __device__ __forceinline__ void load(double* dst, int t, int off, __amdgpu_buffer_rsrc_t r, int z0, int z1,
+                                                int lane)
+    {
+        if constexpr (PAIR) {
+            if (t == 4) ld2_to_lds(r, dst + t * 128, off + (lane < 32 ? z0 : z1), 0);
+            else ld2_to_lds(r, dst + t * 128, off, t < 4 ? z0 : z1);
+        } else {
+            ldw_to_lds(r, dst + t * 32, off, z0);
+            ldw_to_lds(r, dst + PLANE + t * 32, off, z1);
+        }
+    }
+};
+
 template <bool FIRST, bool PAIR>
-__device__ __forceinline__ void rk4_brick_body(const HalfArgs& h, const int bid)
+__device__ __forceinline__ void rk4_brick_body(const HalfArgs& h)
 {
     using B = BrickCfg;
     const FusedArgs& a = h.a;
-    __shared__ __attribute__((aligned(16))) double P[B::D * B::PLANE];
+    __shared__ __attribute__((aligned(16))) double P[2 * B::CELLS];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ni = a.ni, nj = a.nj, nk = a.nk;
-    const int tile = bid % a.tiles;
-    const int chunk = (bid / a.tiles) % a.chunks;
-    const int slice = bid / (a.tiles * a.chunks);
-    const int x0 = (tile % a.tiles_x) * B::BX, y0 = (tile / a.tiles_x) * B::BY, z0 = chunk * B::BZ;
-    const __amdgpu_buffer_rsrc_t rin = make_rsrc((const double*)a.in.p + slice * a.in.slice, a.in_bytes);
-    const __amdgpu_buffer_rsrc_t rq = make_rsrc((const double*)h.q.p + slice * h.q.slice, h.q_bytes);
-    const __amdgpu_buffer_rsrc_t rout = make_rsrc((double*)a.out.p + slice * a.out.slice, a.out_bytes);
-    const int iskb = (int)a.in.sk * 8, qskb = (int)h.q.sk * 8, oskb = (int)a.out.sk * 8;
-    const StarW<double> w = a.cdev ? load_w<double>(a.cdev[slice]) : load_w<double>(a.c);
+    const int iskb = (int)a.in.sk * 8, isj = (int)a.in.sj, qskb = (int)h.q.sk * 8, oskb = (int)a.out.sk * 8;
 
-    brick_load<PAIR, B::W, B::H, B::D>(P, rin, iskb, (int)a.in.sj, x0 - 4, y0 - 4, z0 - 4, ni, nj, nk, wave, lane);
-    // first stage: column 96 zg + s of three planes; s in rows of 8, 10 (eight times), 8 blocks
-    const int za = tid / 96, sa = tid % 96;
-    const int by = sa < 8 ? -1 : sa < 88 ? (sa - 8) / 10 : 8;
-    const int bx = sa < 8 ? sa : sa < 88 ? (sa - 8) % 10 - 1 : sa - 88;
-    double* const ca = P + 3 * za * B::PLANE + (2 * by + 4) * B::W + 2 * bx + 4;
-    d2 qa[3][2];
-    if constexpr (!FIRST) {
-        BrickCols<PAIR> col;
-        col.set(x0 + 2 * bx, y0 + 2 * by, ni, nj, (int)h.q.sj);
+    // this block's bricks: every step-th of its XCD's contiguous range
+    const int xcd = blockIdx.x % 8, extra = h.bricks % 8;
+    const int step = ((int)gridDim.x + 7 - xcd) / 8;
+    const int first = xcd * (h.bricks / 8) + min(xcd, extra), last = first + h.bricks / 8 + (xcd < extra ? 1 : 0);
+    int b = first + (int)blockIdx.x / 8;
+    if (b >= last) return;
+
+    int slice, x0, y0, z0;
+    const auto divide = [](int n, int d, unsigned inv, int& rest) {  // inv: (2^32 - 1) / d
+        int v = (int)__umulhi((unsigned)n, inv);
+        rest = n - v * d;
+        if (rest >= d) ++v, rest -= d;
+        return v;
+    };
+    const auto place = [&](int n) {
+        int tile, chunk, tx;
+        slice = divide(divide(n, a.tiles, h.inv_tiles, tile), a.chunks, h.inv_chunks, chunk);
+        y0 = divide(tile, a.tiles_x, h.inv_tiles_x, tx) * B::BY;
+        x0 = tx * B::BX;
+        z0 = chunk * B::BZ;
+    };
+    const auto input = [&]() { return make_rsrc((const double*)a.in.p + slice * a.in.slice, a.in_bytes); };
+    place(b);
+    using L = BrickLoads<PAIR>;
+    const unsigned span = (unsigned)nk * iskb;
+    {
+        const __amdgpu_buffer_rsrc_t r = input();
+        unsigned z = wrapz(z0 - 4, nk) * iskb;
+        if constexpr (PAIR) {
+            // a part per wave
+            if (wave < L::N) {
+                const int off = L::offset(wave, lane, isj, x0 - 4, y0 - 4, ni, nj);
+                z = wave * 64 + lane < B::PLANE / 2 ? z : L::step(z, iskb, span);
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
+                for (int u = 0; u < B::D / 2; ++u) {
+                    ld2_to_lds(r, P + 2 * u * B::PLANE + wave * 128, off + z, 0);
+                    z = L::step(z, 2 * iskb, span);
+                }
+            }
+        } else if (wave < L::N / 2) {
+            const int off0 = L::offset(2 * wave, lane, isj, x0 - 4, y0 - 4, ni, nj);
+            const int off1 = L::offset(2 * wave + 1, lane, isj, x0 - 4, y0 - 4, ni, nj);
 #pragma unroll
-            for (int f = 0; f < 2; ++f) qa[j][f] = col.ld(rq, f, wrapz(z0 - 2 + 3 * za + j, nk) * qskb);
-    }
-    // second stage: waves 0-3, two planes each
-    const int zb = wave, cx = x0 + 2 * (lane & 7), cy = y0 + 2 * (lane >> 3);
-    d2 qb[2][2];
-    if (wave < 4) {
-        BrickCols<PAIR> col;
-        col.set(cx, cy, ni, nj, (int)h.q.sj);
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int f = 0; f < 2; ++f) qb[j][f] = col.ld(rq, f, wrapz(z0 + 2 * zb + j, nk) * qskb);
-    }
-    vm_wait<0>();
-    lds_barrier();
-    d2 va[3][2];
-    if constexpr (FIRST) brick_stage<3>(va, ca, w, w.f1, nullptr);
-    else brick_stage<3>(va, ca, w, w.f3, qa);
-    lds_barrier();
-#pragma unroll
-    for (int j = 0; j < 3; ++j) quad_write<B::W>(ca + (j + 2) * B::PLANE, va[j]);
-    lds_barrier();
-    if (wave < 4) {
-        const double* const cb = P + (2 * zb + 2) * B::PLANE + (2 * (lane >> 3) + 4) * B::W + 2 * (lane & 7) + 4;
-        d2 vb[2][2];
-        brick_stage<2>(vb, cb, w, FIRST ? w.f2 : w.f4, qb);
-        BrickCols<PAIR> col;
-        col.set(cx, cy, ni, nj, (int)a.out.sj);  // periodic image for partial bricks
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int z = z0 + 2 * zb + j;
-            if (z < nk) {
-#pragma unroll
-                for (int f = 0; f < 2; ++f) col.st(rout, f, z * oskb, vb[j][f]);
+            for (int p = 0; p < B::D; ++p) {
+                ldw_to_lds(r, P + p * B::PLANE + wave * 64, off0, z);
+                ldw_to_lds(r, P + p * B::PLANE + wave * 64 + 32, off1, z);
+                z = L::step(z, iskb, span);
             }
         }
+        vm_wait<0>();
+    }
+
+    if (wave >= B::WAVES) {
+        // the next brick's plane pairs into the other buffer, alternating between the two waves
+        double* dst = P + B::CELLS;
+        for (;;) {
+            const bool more = b + step < last;
+            if (more) place(b + step);
+            const __amdgpu_buffer_rsrc_t r = input();
+            int off[L::N];
+#pragma unroll
+            for (int t = 0; t < L::N; ++t) off[t] = L::offset(t, lane, isj, x0 - 4, y0 - 4, ni, nj);
+            unsigned z = wrapz(z0 - 4 + 2 * (wave - B::WAVES), nk) * iskb;
+            double* d = dst + 2 * (wave - B::WAVES) * B::PLANE;
+            const auto pairs = [&](int n) {
+                if (more)
+                    for (int u = 0; u < n; ++u) {
+                        const unsigned z1 = L::step(z, iskb, span);
+#pragma unroll
+                        for (int t = 0; t < L::N; ++t) L::load(d, t, off[t], r, z, z1, lane);
+                        z = L::step(z, 4 * iskb, span);
+                        d += 4 * B::PLANE;
+                    }
+            };
+            vm_wait<0>();  // the brick that is computed now
+            lds_barrier();
+            pairs(3);
+            lds_barrier();
+            pairs(1);
+            lds_barrier();
+            if (!more) break;
+            b += step;
+            dst = P + (dst == P ? B::CELLS : 0);
+        }
+        return;
+    }
+
+    const StarW<double> w0 = load_w<double>(a.c);
+    // first stage: planes za and za + 1 of twelve of the column (bx, by); the last two waves take
+    // the columns around the brick
+    const int ring = lane & 31;
+    int bx = lane & 7, by = lane >> 3, za = 2 * wave;
+    if (wave >= 6) {
+        bx = ring < 16 ? ring & 7 : ring < 24 ? -1 : 8;
+        by = ring < 8 ? -1 : ring < 16 ? 8 : ring & 7;
+        za = 2 + 4 * (wave - 6) + 2 * (lane >> 5);
+    }
+    double* ca = P + za * B::PLANE + (2 * by + 4) * B::W + 2 * bx + 4;
+    // second stage: a plane per wave
+    const int zb = wave, cx = 2 * (lane & 7), cy = 2 * (lane >> 3);
+    const double* cb = P + (zb + 2) * B::PLANE + (cy + 4) * B::W + cx + 4;
+
+    d2 qa[2][2], qb[1][2];
+    const auto bases = [&]() {  // launch A reads them from the input in LDS
+        if constexpr (!FIRST) {
+            const __amdgpu_buffer_rsrc_t r = make_rsrc((const double*)h.q.p + slice * h.q.slice, h.q_bytes);
+            BrickCols<PAIR> col;
+            col.set(x0 + 2 * bx, y0 + 2 * by, ni, nj, (int)h.q.sj);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int f = 0; f < 2; ++f) qa[j][f] = col.ld_lane(r, f, wrapz(z0 - 2 + za + j, nk) * qskb);
+            col.set(x0 + cx, y0 + cy, ni, nj, (int)h.q.sj);
+#pragma unroll
+            for (int f = 0; f < 2; ++f) qb[0][f] = col.ld(r, f, wrapz(z0 + zb, nk) * qskb);
+        }
+    };
+    bases();
+    int next = B::CELLS;
+    for (;;) {
+        lds_barrier();
+        const StarW<double> w = a.cdev ? load_w<double>(a.cdev[slice]) : w0;
+        d2 va[2][2];
+        if constexpr (FIRST) {
+            brick_stage<2>(va, ca, w, w.f1, nullptr);
+            quad_read_c<B::W>(cb + 2 * B::PLANE, qb[0]);
+        } else {
+            brick_stage<2>(va, ca, w, w.f3, qa);
+        }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) quad_write<B::W>(ca + (j + 2) * B::PLANE, va[j]);
+        lds_barrier();
+        d2 vb[1][2];
+        brick_stage<1>(vb, cb, w, FIRST ? w.f2 : w.f4, qb);
+        if (z0 + zb < nk) {
+            const __amdgpu_buffer_rsrc_t r = make_rsrc((double*)a.out.p + slice * a.out.slice, a.out_bytes);
+            BrickCols<PAIR> col;
+            col.set(x0 + cx, y0 + cy, ni, nj, (int)a.out.sj);  // periodic image for partial bricks
+#pragma unroll
+            for (int f = 0; f < 2; ++f) col.st(r, f, (z0 + zb) * oskb, vb[0][f]);
+        }
+        if (b + step >= last) break;
+        b += step;
+        place(b);
+        bases();
+        ca += next;
+        cb += next;
+        next = -next;
     }
 }
 
@@ -1646,9 +1786,9 @@ __global__ void __launch_bounds__(NT) k_rk4_half_pair(HalfArgs h)
 }
 
 template <bool FIRST, bool PAIR>
-__global__ void __launch_bounds__(BrickCfg::NT, 3) k_rk4_brick(HalfArgs h)
+__global__ void __launch_bounds__(BrickCfg::THREADS) k_rk4_brick(HalfArgs h)
 {
-    rk4_brick_body<FIRST, PAIR>(h, xcd_block(blockIdx.x, gridDim.x));
+    rk4_brick_body<FIRST, PAIR>(h);
 }
 
 // One launch over several independent batches (problems of different sizes, steps and
@@ -1831,16 +1971,24 @@ int launch_split(hipStream_t s, const FusedStep& st, const FusedTile& tile, View
     SP_TRY(fill_args(B.a, st, tile, wv, out, 8, 8));
     B.q = in;
     B.q_bytes = A.a.in_bytes;
-    const dim3 grid(nblocks_of(A.a, st.nslices));
+    dim3 grid(nblocks_of(A.a, st.nslices));
     if (is_brick(tile)) {
+        for (HalfArgs* h : {&A, &B}) {
+            h->bricks = (int)grid.x;
+            h->inv_tiles = 0xffffffffu / h->a.tiles;
+            h->inv_chunks = 0xffffffffu / h->a.chunks;
+            h->inv_tiles_x = 0xffffffffu / h->a.tiles_x;
+        }
+        grid.x = std::min(grid.x, 256u);  // two buffers fill a CU's LDS: one block per CU
+        const dim3 block(BrickCfg::THREADS);
         // each launch by its own fields' alignment (the work field's rows are ni long)
         const bool even = (st.ni & 1) == 0;
-        if (even && pair_ok(st, in, wv)) hipLaunchKernelGGL((k_rk4_brick<true, true>), grid, dim3(BrickCfg::NT), 0, s, A);
-        else hipLaunchKernelGGL((k_rk4_brick<true, false>), grid, dim3(BrickCfg::NT), 0, s, A);
+        if (even && pair_ok(st, in, wv)) hipLaunchKernelGGL((k_rk4_brick<true, true>), grid, block, 0, s, A);
+        else hipLaunchKernelGGL((k_rk4_brick<true, false>), grid, block, 0, s, A);
         SP_HIP(hipGetLastError());
         if (even && pair_ok(st, in, wv) && pair_ok(st, wv, out))
-            hipLaunchKernelGGL((k_rk4_brick<false, true>), grid, dim3(BrickCfg::NT), 0, s, B);
-        else hipLaunchKernelGGL((k_rk4_brick<false, false>), grid, dim3(BrickCfg::NT), 0, s, B);
+            hipLaunchKernelGGL((k_rk4_brick<false, true>), grid, block, 0, s, B);
+        else hipLaunchKernelGGL((k_rk4_brick<false, false>), grid, block, 0, s, B);
         SP_HIP(hipGetLastError());
         return SP_OK;
     }
@@ -2010,20 +2158,21 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
     //   2x2: 1.25-1.4 per plane and round of 256 blocks (1 x 256^3 in 64-plane chunks 120, 4 x
     //   128^3 in 32-plane chunks 73, 16 x 128^3 210, 1 x 384^3 in 128-plane chunks 389); the
     //   whole-k and 64-plane chunks chosen before: 1 x 256^3 250, 4 x 128^3 155, 1 x 384^3 437.
-    //   bricks: 14 up to 256 of them, then 8 + 0.033 each (1 x 64^3 14.1 against 35 for the 2x2
-    //   kernel; 432 bricks, 1 x 96^3: 23 against 35; 1024, 1 x 128^3: 41 against 36).
-    // Odd x extents cannot take the 2x2 kernel's 16-byte accesses: bricks (0.055 each; 1024
-    // bricks, 127^3: 56) or the scalar kernel (127^3 56, 161^3 148 in 64-plane chunks against 145 for
-    // bricks, 255^3 287 against 441).
+    //   bricks: 8.3 and 5.8 per round of 256 (1 x 64^3 13.2 against 35 for the 2x2 kernel; 432
+    //   bricks, 1 x 96^3: 21 against 35; 1024, 1 x 128^3: 32.5 against 35.3; 1728, 4 x 96^3: 48
+    //   against 41).
+    // Odd x extents cannot take the 2x2 kernel's 16-byte accesses: bricks, 8.1 per round, while
+    // they are not slower than the scalar kernel (127^3 40 against 56, 161^3 84 against 145, 201^3
+    // 141 against 271, 255^3, 8192 bricks, 284 against 287).
     const long long bricks = tiles_of(ni, nj, nslices, 16, 16) * ((nk + 7) / 8);
     if (compute_f64 && !one_launch) {
         const FusedTile brick{16, 16, 384, 8, SP_KERNEL_SPLIT};
         if (ni & 1) {
-            if (bricks <= 2048) return brick;
+            if (bricks <= 8192) return brick;
         } else {
             double us;
             const int kc = best_kchunk(tiles_of(ni, nj, nslices, 32, 32), nk, kQuadWalk, &us);
-            if (std::max(14., 8. + 0.033 * bricks) < us) return brick;
+            if (8.3 + 5.8 * ((bricks + 255) / 256) < us) return brick;
             return FusedTile{32, 32, 512, kc >= nk ? 0 : kc, SP_KERNEL_QUAD};
         }
     }

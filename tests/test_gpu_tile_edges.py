@@ -54,3 +54,20 @@ def test_brick_kernel_edges(sp, shape):
     assert np.array_equal(got, ref)
     exact = O.OConvection(*shape, 1. / 32, 0.02, 30.0, *C3).rk4(q0, 0.0, 1e-4, 4)
     assert np.abs(got - exact).max() <= 1e-12 * np.abs(exact).max()
+
+
+@pytest.mark.parametrize("shape", [(96, 98, 72), (145, 131, 40), (272, 258, 17)], ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("kind", ["compact", "stella"])
+def test_bricks_in_turn(sp, shape, kind):
+    """More bricks than blocks: 378 to 867, the last ones partial in every direction."""
+    ni, nj, nk = shape
+    q0 = np.random.default_rng(ni).standard_normal((nk, nj, ni))
+    out = []
+    for variant, tile, kchunk in (("scalar", (32, 16, 512), 0), ("split", (16, 16, 384), 8)):
+        conv = sp.Convection(ni, nj, nk, 1. / 64, 0.02, 0.0, *C3)
+        conv.set_tile(*tile, kchunk, variant=variant)
+        a, b = conv.field(kind=kind), conv.field(kind=kind)
+        a.set(q0)
+        conv.DoRK4(a, b, 0.0, 1e-4, 3)
+        out.append(b.get())
+    assert np.isfinite(out[0]).all() and np.array_equal(*out)
