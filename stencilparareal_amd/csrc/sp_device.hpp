@@ -21,6 +21,12 @@ __device__ __forceinline__ int near_mod(int a, int n)
     return a - (a >= n ? n : 0);
 }
 
+// z, a plane's byte offset below span (all planes'), d <= span further on
+__device__ __forceinline__ unsigned plane_step(unsigned z, unsigned d, unsigned span)
+{
+    return min(z + d, z + d - span);  // the second is huge unless the first is past the end
+}
+
 // Plane index p in [-3n, 4n) wrapped into [0, n) without branches (scalar selects).  The
 // stream touches planes z0-18 .. zend+16, inside that range for n >= 8; the host sends
 // smaller k extents to the reference-order path.
@@ -71,8 +77,9 @@ template <int N>
 __device__ __forceinline__ void vm_wait() { __builtin_amdgcn_s_waitcnt(0x0F70 | N); }
 
 // Workgroup barrier for LDS data: this wave's LDS accesses are complete before it, but for the
-// last N issued (reads of planes that nobody writes next), and none moves across it.  Unlike __syncthreads it leaves loads into LDS in flight (vm_wait before it
-// for those that another wave reads next).
+// last N issued (reads of planes that nobody writes next), and none moves across it.  Unlike
+// __syncthreads it leaves loads into LDS in flight (vm_wait before it for those that another wave
+// reads next).
 template <int N = 0>
 __device__ __forceinline__ void lds_barrier()
 {
@@ -84,33 +91,30 @@ __device__ __forceinline__ void lds_barrier()
 }
 
 // Loads a brick of D planes of H rows of W doubles (W even, at most 640 cells per plane) from
-// (x, y, z) on (x and y at most 24 cells outside the field), with periodic images, into P in the order of its cells, straight into LDS: a
-// plane's 16-byte slots by the lanes of waves 0 to 4, or (not PAIR: rows that are not 16-byte
-// aligned pairs) four words per lane.  The caller waits for the loads (vm_wait, barrier).
+// (x, y, z) on (x and y at most 24 cells outside the field), with periodic images, into P in the
+// order of its cells, straight into LDS: a plane's 16-byte slots by the lanes of waves 0 to 4, or
+// (not PAIR: rows that are not 16-byte aligned pairs) four words per lane.  The caller waits for
+// the loads (vm_wait, barrier).
 template <bool PAIR, int W, int H, int D>
 __device__ __forceinline__ void brick_load(double* P, __amdgpu_buffer_rsrc_t r, int skb, int sj, int x, int y, int z,
                                            int ni, int nj, int nk, int wave, int lane)
 {
     static_assert(W % 2 == 0 && W * H <= 640, "five waves' slots hold a plane");
     if (wave >= 5) return;
-    constexpr int M = PAIR ? 1 : 4;
-    int off[M];
-    bool in[M];
+    const unsigned span = (unsigned)nk * skb, zo = wrapz(z, nk) * skb;
+    // one mask for all planes of a lane's cell: masks and scalar work around each load would
+    // cost more than the load
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
+    for (int m = 0; m < (PAIR ? 1 : 4); ++m) {
         const int e = PAIR ? 2 * (wave * 64 + lane) : wave * 128 + m * 32 + (lane >> 1);  // cell of the plane
-        in[m] = e < W * H;
-        off[m] = (near_mod(x + e % W, ni) + near_mod(y + e / W, nj) * sj) * 8 + (PAIR ? 0 : (lane & 1) * 4);
-    }
+        if (e < W * H) {
+            const int off = (near_mod(x + e % W, ni) + near_mod(y + e / W, nj) * sj) * 8 + (PAIR ? 0 : (lane & 1) * 4);
+            double* const dst = P + wave * 128 + m * 32;
+            unsigned o = zo;
 #pragma unroll
-    for (int p = 0; p < D; ++p) {
-        const int zo = wrapz(z + p, nk) * skb;
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            double* const dst = P + p * W * H + wave * 128 + m * 32;
-            if (in[m]) {
-                if constexpr (PAIR) ld2_to_lds(r, dst, off[m], zo);
-                else ldw_to_lds(r, dst, off[m], zo);
+            for (int p = 0; p < D; ++p, o = plane_step(o, skb, span)) {
+                if constexpr (PAIR) ld2_to_lds(r, dst + p * W * H, off, o);
+                else ldw_to_lds(r, dst + p * W * H, off, o);
             }
         }
     }

@@ -1578,11 +1578,6 @@ struct BrickLoads {
         const int e = PAIR ? (2 * (t * 64 + lane)) % PLANE : t * 32 + (lane >> 1);
         return (near_mod(x + e % W, ni) + near_mod(y + e / W, nj) * sj) * 8 + (PAIR ? 0 : (lane & 1) * 4);
     }
-    // z, a plane's byte offset below span (all planes'), d < span further on
-    static __device__ __forceinline__ unsigned step(unsigned z, unsigned d, unsigned span)
-    {
-        return min(z + d, z + d - span);  // the second is huge unless the first is past the end
-    }
     // part t of the plane pair at dst, planes at byte offsets z0 and z1
     static __device__ __forceinline__ void load(double* dst, int t, int off, __amdgpu_buffer_rsrc_t r, int z0, int z1,
                                                 int lane)
@@ -1641,11 +1636,11 @@ __device__ __forceinline__ void rk4_brick_body(const HalfArgs& h)
             // a part per wave
             if (wave < L::N) {
                 const int off = L::offset(wave, lane, isj, x0 - 4, y0 - 4, ni, nj);
-                z = wave * 64 + lane < B::PLANE / 2 ? z : L::step(z, iskb, span);
+                z = wave * 64 + lane < B::PLANE / 2 ? z : plane_step(z, iskb, span);
 #pragma unroll
                 for (int u = 0; u < B::D / 2; ++u) {
                     ld2_to_lds(r, P + 2 * u * B::PLANE + wave * 128, off + z, 0);
-                    z = L::step(z, 2 * iskb, span);
+                    z = plane_step(z, 2 * iskb, span);
                 }
             }
         } else if (wave < L::N / 2) {
@@ -1655,7 +1650,7 @@ __device__ __forceinline__ void rk4_brick_body(const HalfArgs& h)
             for (int p = 0; p < B::D; ++p) {
                 ldw_to_lds(r, P + p * B::PLANE + wave * 64, off0, z);
                 ldw_to_lds(r, P + p * B::PLANE + wave * 64 + 32, off1, z);
-                z = L::step(z, iskb, span);
+                z = plane_step(z, iskb, span);
             }
         }
         vm_wait<0>();
@@ -1676,10 +1671,10 @@ __device__ __forceinline__ void rk4_brick_body(const HalfArgs& h)
             const auto pairs = [&](int n) {
                 if (more)
                     for (int u = 0; u < n; ++u) {
-                        const unsigned z1 = L::step(z, iskb, span);
+                        const unsigned z1 = plane_step(z, iskb, span);
 #pragma unroll
                         for (int t = 0; t < L::N; ++t) L::load(d, t, off[t], r, z, z1, lane);
-                        z = L::step(z, 4 * iskb, span);
+                        z = plane_step(z, 4 * iskb, span);
                         d += 4 * B::PLANE;
                     }
             };

@@ -216,7 +216,7 @@ __device__ __forceinline__ void euler_brick_step(const EulerBrick& a, double* P,
     } else if (live) {
         const int oskb = (int)a.out.sk * 8;
         // periodic image for partial bricks
-        const int o = (pmod(x0 + x, a.P.ni) + pmod(y0 + y, a.P.nj) * (int)a.out.sj) * 8;
+        const int o = (near_mod(x0 + x, a.P.ni) + near_mod(y0 + y, a.P.nj) * (int)a.out.sj) * 8;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             const int z = z0 + half * N + j;
