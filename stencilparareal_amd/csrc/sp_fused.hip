@@ -1496,10 +1496,10 @@ __device__ __forceinline__ void rk4_quad_body(const FusedArgs& a, const int bid)
 // alignment: PAIR loads and stores 16 bytes, otherwise each cell's two words are loaded by
 // lanes of their own.  Eight columns per row and a row pair of 24 chunks of 16 bytes (8 mod 16)
 // put consecutive lanes on consecutive chunks across rows: no bank conflicts.
-// Bound by latency up to 256 bricks (64^3 13.2 us a step), then by memory accesses in flight:
-// 2.9 us per brick and launch, of which loads and stores alone take 2.6 and the stages 1.8.  One
-// brick per block on six waves, loads not overlapped: 64^3 13.9, 128^3 42.0 against 32.5 us, 127^3
-// 52.4 against 40.4, 8 x 64^3 40.3 against 32.1.
+// Bound by latency up to 256 bricks (64^3 13.0 us a step), then by no one part alone: 128^3, 1024
+// bricks, took 32.4 us, without its loads 32.6, without its stores 27 (30.5 since these go
+// through), without the two stages 28, without all of them 18.  One brick per block on six waves,
+// loads not overlapped: 64^3 13.9 us, 128^3 42.0, 127^3 52.4 against 40.4, 8 x 64^3 40.3 against 29.5.
 struct BrickCfg {
     static constexpr int BX = 16, BY = 16, BZ = 8, NT = 384;  // NT: the descriptor's only
     static constexpr int W = 24, H = 24, D = 16, PLANE = W * H, CELLS = D * PLANE;  // the input's cells in LDS
@@ -1531,9 +1531,9 @@ struct BrickCols {
     __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, int f, int zo, d2 v) const
     {
         if constexpr (PAIR) {
-            st2(r, o[f][0], zo, v);
+            st_through(r, o[f][0], zo, v);
         } else {
-            Buf<double>::st(r, o[f][0], zo, v.x);
+            Buf<double>::st(r, o[f][0], zo, v.x);  // halves of lines: 10 % slower stored through
             Buf<double>::st(r, o[f][1], zo, v.y);
         }
     }
@@ -2153,8 +2153,8 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
     //   2x2: 1.25-1.4 per plane and round of 256 blocks (1 x 256^3 in 64-plane chunks 120, 4 x
     //   128^3 in 32-plane chunks 73, 16 x 128^3 210, 1 x 384^3 in 128-plane chunks 389); the
     //   whole-k and 64-plane chunks chosen before: 1 x 256^3 250, 4 x 128^3 155, 1 x 384^3 437.
-    //   bricks: 8.3 and 5.8 per round of 256 (1 x 64^3 13.2 against 35 for the 2x2 kernel; 432
-    //   bricks, 1 x 96^3: 21 against 35; 1024, 1 x 128^3: 32.5 against 35.3; 1728, 4 x 96^3: 48
+    //   bricks: 7.5 and 5.7 per round of 256 (1 x 64^3 13.0 against 35 for the 2x2 kernel; 432
+    //   bricks, 1 x 96^3: 19 against 35; 1024, 1 x 128^3: 30.5 against 35.3; 1728, 4 x 96^3: 46
     //   against 41).
     // Odd x extents cannot take the 2x2 kernel's 16-byte accesses: bricks, 8.1 per round, while
     // they are not slower than the scalar kernel (127^3 40 against 56, 161^3 84 against 145, 201^3
@@ -2167,7 +2167,7 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
         } else {
             double us;
             const int kc = best_kchunk(tiles_of(ni, nj, nslices, 32, 32), nk, kQuadWalk, &us);
-            if (8.3 + 5.8 * ((bricks + 255) / 256) < us) return brick;
+            if (7.5 + 5.7 * ((bricks + 255) / 256) < us) return brick;
             return FusedTile{32, 32, 512, kc >= nk ? 0 : kc, SP_KERNEL_QUAD};
         }
     }

@@ -160,8 +160,8 @@ __global__ void __launch_bounds__(256) k_euler_fused(StagedParams P, Spacing d, 
 // step's results wait in registers until every lane has read, then replace the field in LDS.
 // Each point is the expression of DoEulerTimestep (Convection.cpp:372-392) in the reference's
 // order: the same bits as two launches.  Where dx is a power of two the two divisions are
-// products (the same numbers).  Measured per step, before and now: 96^3 9.0 -> 6.0 us, 128^3
-// 12.3 -> 7.4, 192^3 34 -> 26, 256^3 79 -> 42, 384^3 318 -> 198; 64^3 and smaller are bound by the
+// products (the same numbers).  Measured per step, before and now: 96^3 9.0 -> 5.6 us, 128^3
+// 12.3 -> 6.4, 192^3 34 -> 25, 256^3 79 -> 40, 384^3 318 -> 193; 64^3 and smaller are bound by the
 // launches.  Three and four steps per launch were slower from 96^3 on (128^3 8.5 and 8.7 us, 384^3
 // 241 and 258): 1.9 and 2.5 times the points' operations.
 struct EulerBrick {
@@ -220,9 +220,7 @@ __device__ __forceinline__ void euler_brick_step(const EulerBrick& a, double* P,
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             const int z = z0 + half * N + j;
-            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-            if (z < a.P.nk)
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, r[j]), rout, o + z * oskb, 0, 0);
+            if (z < a.P.nk) st_through(rout, o + z * oskb, 0, r[j]);
         }
     }
 }
