@@ -154,6 +154,24 @@ int ensure_split(sp_prop* p, const FusedTile& t, int nslices)
     return p->split.ensure(split_work_bytes(p->ni, p->nj, p->nk, nslices));
 }
 
+// The tile of a step's call, its work field there.  A built-in choice needs nothing that the call
+// would not have held without it: where the call keeps no scratch (and so may be captured cold, or
+// run on several streams at once) or there is no memory for the work field, it is the one-launch
+// tile (the same bits).
+int call_tile(sp_prop* p, int nslices, int f64, bool scratch, FusedTile* t)
+{
+    *t = pick_tile(p, nslices, f64);
+    if (t->variant != SP_KERNEL_SPLIT) return SP_OK;
+    const bool builtin = p->tile.tx == 0 && !p->tuned.count({nslices, f64 ? 1 : 0});
+    if (scratch || !builtin) {
+        const int r = ensure_split(p, *t, nslices);
+        if (r == SP_OK || !builtin) return r;
+        (void)hipGetLastError();  // the allocation's
+    }
+    *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, true);
+    return SP_OK;
+}
+
 // Autotuner: times every candidate tile / k chunk of the fused kernel for `nslices` slices
 // (views in -> out, slice stride set) and records the fastest for pick_tile.  Synchronous;
 // refuses to run while the stream is being captured.
@@ -294,8 +312,8 @@ int rk4_fused_run(sp_prop* p, int idt, View vin, int odt, View vout, bool aliase
     const size_t bytes = n * dtype_size(sdt);
     SP_TRY(p->scratch[0].ensure(bytes));
     if (aliased) SP_TRY(p->scratch[1].ensure(bytes));
-    const FusedTile tile = pick_tile(p, 1, idt == SP_F64 && odt == SP_F64);
-    SP_TRY(ensure_split(p, tile, 1));
+    FusedTile tile;
+    SP_TRY(call_tile(p, 1, idt == SP_F64 && odt == SP_F64, true, &tile));
     const View A = cview(p->scratch[0].p, p->ni, p->nj), B = cview(p->scratch[1].p, p->ni, p->nj);
     View src = vin;
     int sdtype = idt;
@@ -768,8 +786,8 @@ int sp_do_rk4_batched(sp_prop* p, int nslices, const sp_layout* lin, const void*
         SP_TRY(p->scratch[0].ensure(bytes));
         A.p = (char*)p->scratch[0].p + lout->origin * dtype_size(lout->dtype);
     }
-    const FusedTile tile = pick_tile(p, nslices, lin->dtype == SP_F64 && lout->dtype == SP_F64);
-    SP_TRY(ensure_split(p, tile, nslices));
+    FusedTile tile;
+    SP_TRY(call_tile(p, nslices, lin->dtype == SP_F64 && lout->dtype == SP_F64, steps > 1, &tile));
     View cur = vin;
     int cdt = lin->dtype;
     for (int i = 0; i < steps; ++i) {

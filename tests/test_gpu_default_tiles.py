@@ -37,3 +37,33 @@ def test_default_tile(sp, shape, storage):
         conv.DoRK4(a, b, 0.0, 1e-4, 3)
         out.append(b.get())
     assert np.isfinite(out[1]).all() and np.array_equal(*out)
+
+
+def test_single_batched_step_keeps_no_scratch(sp):
+    """A batched call of one step holds nothing between its input and output: captured before any
+    other call, each replay gives the bits of the scalar kernel, on inputs changed in between."""
+    import ctypes as C
+    from stencilparareal_amd import _lib as L
+
+    n, S = 32, 3
+    lay = L.Layout()
+    L.call("sp_layout_compact", n, n, n, 0, C.byref(lay))
+
+    def step(conv, a, b):
+        conv.ctx.sync_stream()
+        L.call("sp_do_rk4_batched", conv.h, S, C.byref(lay), C.c_void_p(a.data_ptr()), C.byref(lay),
+               C.c_void_p(b.data_ptr()), n**3, 0.0, 1e-4, 1)
+
+    conv, ref = (sp.Convection(n, n, n, 1. / n, 0.02, 0.0, 1.0, -0.5, 0.25) for _ in range(2))
+    ref.set_tile(32, 16, 512, 0, variant="scalar")
+    a = torch.empty(S, n, n, n, dtype=torch.float64, device="cuda")
+    b, want = torch.empty_like(a), torch.empty_like(a)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        step(conv, a, b)
+    for seed in range(3):
+        a.copy_(torch.from_numpy(np.random.default_rng(seed).standard_normal((S, n, n, n))))
+        g.replay()
+        step(ref, a, want)
+        torch.cuda.synchronize()
+        assert torch.equal(b, want)
