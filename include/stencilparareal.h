@@ -126,9 +126,10 @@ int sp_prop_set_path(sp_prop* p, int path);
  * 32x16x512, 32x16x256, 16x16x256, 16x16x384}.  The split variant (FP64 fields) runs each
  * step as two launches through a work field the propagator allocates (8 bytes per point
  * of the batch) when the tile is chosen; its results equal the other FP64 variants' bit
- * for bit.  Its shape 16x16x384 computes bricks of 16x16x8 points (whatever kchunk says), on
- * any sizes and strides; the other shapes need an even ni.  Grouped batches (sp_batch_*) and sp_do_rk4_noalloc run the built-in FP64
- * choice in its place. */
+ * for bit.  Its shape 16x16x384 computes bricks of 16x16x8 points (whatever kchunk says, in
+ * blocks of 640 threads), on any sizes and strides; the other shapes need an even ni.  Grouped
+ * batches (sp_batch_*) and sp_do_rk4_noalloc run the built-in one-launch choice in its place, as
+ * does a built-in choice in a batched call of one step or without memory for the work field. */
 int sp_prop_set_tile(sp_prop* p, int variant, int tx, int ty, int nthreads, int kchunk);
 /* The fused-kernel tile sp_do_rk4 (nslices = 1) or sp_do_rk4_batched (nslices > 1) will
  * use for FP64 compute (f64 = 1) or reduced-precision storage (f64 = 0): the one set with
