@@ -158,11 +158,13 @@ int ensure_split(sp_prop* p, const FusedTile& t, int nslices)
 // would not have held without it: where the call keeps no scratch (and so may be captured cold, or
 // run on several streams at once) or there is no memory for the work field, it is the one-launch
 // tile (the same bits).
-int call_tile(sp_prop* p, int nslices, int f64, bool scratch, FusedTile* t)
+int call_tile(sp_prop* p, int nslices, int f64, bool scratch, bool aligned, FusedTile* t)
 {
     *t = pick_tile(p, nslices, f64);
-    if (t->variant != SP_KERNEL_SPLIT) return SP_OK;
     const bool builtin = p->tile.tx == 0 && !p->tuned.count({nslices, f64 ? 1 : 0});
+    if (builtin && !aligned && p->tile.kchunk < 0)
+        *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, false, false);
+    if (t->variant != SP_KERNEL_SPLIT) return SP_OK;
     if (scratch || !builtin) {
         const int r = ensure_split(p, *t, nslices);
         if (r == SP_OK || !builtin) return r;
@@ -170,6 +172,12 @@ int call_tile(sp_prop* p, int nslices, int f64, bool scratch, FusedTile* t)
     }
     *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, true);
     return SP_OK;
+}
+
+// Whether a view's x pairs are aligned accesses of two elements.
+bool pairs_aligned(const View& v, int dtype)
+{
+    return ((v.sj | v.sk | v.slice) & 1) == 0 && (uintptr_t)v.p % (2 * dtype_size(dtype)) == 0;
 }
 
 // Autotuner: times every candidate tile / k chunk of the fused kernel for `nslices` slices
@@ -313,7 +321,9 @@ int rk4_fused_run(sp_prop* p, int idt, View vin, int odt, View vout, bool aliase
     SP_TRY(p->scratch[0].ensure(bytes));
     if (aliased) SP_TRY(p->scratch[1].ensure(bytes));
     FusedTile tile;
-    SP_TRY(call_tile(p, 1, idt == SP_F64 && odt == SP_F64, true, &tile));
+    // later steps run between the output and the scratch, whose rows are ni long
+    const bool aligned = pairs_aligned(vout, odt) && (steps > 1 || pairs_aligned(vin, idt));
+    SP_TRY(call_tile(p, 1, idt == SP_F64 && odt == SP_F64, true, aligned, &tile));
     const View A = cview(p->scratch[0].p, p->ni, p->nj), B = cview(p->scratch[1].p, p->ni, p->nj);
     View src = vin;
     int sdtype = idt;
@@ -713,6 +723,8 @@ int sp_do_rk4_noalloc(sp_prop* p, const sp_layout* lin, const void* in, const sp
     const bool aliased = same_origin(lin, in, lout, out);
     const View A = cview(g_noalloc_ptr[dev], p->ni, p->nj);
     FusedTile tile = pick_tile(p, 1, 1);
+    if (p->tile.tx == 0 && p->tile.kchunk < 0 && !p->tuned.count({1, 1}) && !pairs_aligned(vout, SP_F64))
+        tile = default_tile(p->ni, p->nj, p->nk, 1, 1, true);
     // the split steps need a second intermediate field: the built-in one-launch tile instead
     // (the same result bit for bit)
     if (tile.variant == SP_KERNEL_SPLIT) tile = default_tile(p->ni, p->nj, p->nk, 1, 1, true);
@@ -787,7 +799,8 @@ int sp_do_rk4_batched(sp_prop* p, int nslices, const sp_layout* lin, const void*
         A.p = (char*)p->scratch[0].p + lout->origin * dtype_size(lout->dtype);
     }
     FusedTile tile;
-    SP_TRY(call_tile(p, nslices, lin->dtype == SP_F64 && lout->dtype == SP_F64, steps > 1, &tile));
+    const bool aligned = pairs_aligned(vout, lout->dtype) && (steps > 1 || pairs_aligned(vin, lin->dtype));
+    SP_TRY(call_tile(p, nslices, lin->dtype == SP_F64 && lout->dtype == SP_F64, steps > 1, aligned, &tile));
     View cur = vin;
     int cdt = lin->dtype;
     for (int i = 0; i < steps; ++i) {

@@ -2146,8 +2146,9 @@ int best_kchunk(long long tiles, int nk, const WalkCost& c, double* us)
 
 }  // namespace
 
-FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, bool one_launch)
+FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, bool one_launch, bool aligned)
 {
+    const bool pairs = aligned && !(ni & 1);  // rows of aligned x pairs
     // FP64: the 2x2 kernel with the k chunk that finishes first, or bricks (two launches) while
     // those are few.  Measured on MI355X in us per step:
     //   2x2: 1.25-1.4 per plane and round of 256 blocks (1 x 256^3 in 64-plane chunks 120, 4 x
@@ -2156,14 +2157,15 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
     //   bricks: 7.5 and 5.7 per round of 256 (1 x 64^3 13.0 against 35 for the 2x2 kernel; 432
     //   bricks, 1 x 96^3: 19 against 35; 1024, 1 x 128^3: 30.5 against 35.3; 1728, 4 x 96^3: 46
     //   against 41).
-    // Odd x extents cannot take the 2x2 kernel's 16-byte accesses: bricks, 8.1 per round, while
-    // they are not slower than the scalar kernel (127^3 40 against 56, 161^3 84 against 145, 201^3
-    // 141 against 271, 255^3, 8192 bricks, 284 against 287).
+    // Odd x extents and strides cannot take the 2x2 kernel's 16-byte accesses: bricks, 8.1 per
+    // round, while they are faster than the scalar kernel (127^3 40 against 56, 161^3 84 against
+    // 145, 201^3 141 against 271; 255^3, 8192 bricks, 284 against 287, and 256^3 in rows of 257
+    // 267 for the scalar kernel).
     const long long bricks = tiles_of(ni, nj, nslices, 16, 16) * ((nk + 7) / 8);
     if (compute_f64 && !one_launch) {
         const FusedTile brick{16, 16, 384, 8, SP_KERNEL_SPLIT};
-        if (ni & 1) {
-            if (bricks <= 8192) return brick;
+        if (!pairs) {
+            if (bricks < 8192) return brick;
         } else {
             double us;
             const int kc = best_kchunk(tiles_of(ni, nj, nslices, 32, 32), nk, kQuadWalk, &us);
@@ -2176,7 +2178,7 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
     // round of two and more, 16x16 0.88 and 0.60.  1 x 64^3 16x16 in 8-plane chunks 23.6 us (34.5
     // for 32x16 in 16), 1 x 256^3 32x32 in 64 122 (154 for 32x16 in 128), 1 x 384^3 32x32 in 77-80
     // 435 (479 in 64; BF16 526 against 598, its best, 32x16 in 64, 499).
-    if (!compute_f64 && !one_launch && !(ni & 1)) {
+    if (!compute_f64 && !one_launch && pairs) {
         static constexpr struct {
             int tx, ty, nt;
             WalkCost cost;

@@ -190,7 +190,8 @@ bool fused_tile_supported(const FusedTile& t, int compute_f64);
 // The split variant's brick shape: any sizes and alignment.
 bool fused_tile_brick(const FusedTile& t);
 // The built-in choice; one_launch: of the kernels that step in one launch without a work field.
-FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, bool one_launch = false);
+FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, bool one_launch = false,
+                       bool aligned = true);
 // Grouped launches: one launch over several batches with their own sizes, views, steps and
 // coefficients.  fused_record_fill writes the kernel's argument record for one batch (of
 // fused_record_size() bytes) and its block count; the caller uploads the records and the

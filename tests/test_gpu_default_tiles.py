@@ -67,3 +67,28 @@ def test_single_batched_step_keeps_no_scratch(sp):
         step(ref, a, want)
         torch.cuda.synchronize()
         assert torch.equal(b, want)
+
+
+@pytest.mark.parametrize("n", [32, 90, 130])
+@pytest.mark.parametrize("steps", [1, 2])
+def test_default_tile_odd_rows(sp, n, steps):
+    """Rows of n + 1 doubles, n even: no aligned x pairs in the output."""
+    import ctypes as C
+    from stencilparareal_amd import _lib as L
+
+    lay = L.Layout()
+    L.call("sp_layout_compact", n, n, n, 0, C.byref(lay))
+    lay.sj, lay.sk = n + 1, (n + 1) * n
+    a = torch.from_numpy(np.random.default_rng(n).standard_normal((n, n, n + 1))).cuda()
+    out = []
+    for tile in (None, (32, 16, 512, 0)):
+        conv = sp.Convection(n, n, n, 1. / 64, 0.02, 0.0, 1.0, -0.5, 0.25)
+        if tile:
+            conv.set_tile(*tile, variant="scalar")
+        b = torch.zeros_like(a)
+        conv.ctx.sync_stream()
+        L.call("sp_do_rk4", conv.h, C.byref(lay), C.c_void_p(a.data_ptr()), C.byref(lay), C.c_void_p(b.data_ptr()),
+               0.0, 1e-4, steps)
+        torch.cuda.synchronize()
+        out.append(b)
+    assert torch.isfinite(out[1]).all() and torch.equal(*out)
