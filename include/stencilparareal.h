@@ -129,7 +129,9 @@ int sp_prop_set_path(sp_prop* p, int path);
  * for bit.  Its shape 16x16x384 computes bricks of 16x16x8 points (whatever kchunk says, in
  * blocks of 640 threads), on any sizes and strides; the other shapes need an even ni.  Grouped
  * batches (sp_batch_*) and sp_do_rk4_noalloc run the built-in one-launch choice in its place, as
- * does a built-in choice in a batched call of one step or without memory for the work field. */
+ * do calls without a tile set where there is no memory for the work field, and those of a single
+ * step with in != out, which use nothing but in and out: calls of that kind may run on several
+ * streams at once, and a captured one stays valid whatever the propagator runs later. */
 int sp_prop_set_tile(sp_prop* p, int variant, int tx, int ty, int nthreads, int kchunk);
 /* The fused-kernel tile sp_do_rk4 (nslices = 1) or sp_do_rk4_batched (nslices > 1) will
  * use for FP64 compute (f64 = 1) or reduced-precision storage (f64 = 0): the one set with

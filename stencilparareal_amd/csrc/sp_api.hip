@@ -154,20 +154,20 @@ int ensure_split(sp_prop* p, const FusedTile& t, int nslices)
     return p->split.ensure(split_work_bytes(p->ni, p->nj, p->nk, nslices));
 }
 
-// The tile of a step's call, its work field there.  A built-in choice needs nothing that the call
-// would not have held without it: where the call keeps no scratch (and so may be captured cold, or
-// run on several streams at once) or there is no memory for the work field, it is the one-launch
-// tile (the same bits).
+// The tile of a step's call, its work field there.  Unless the caller set the tile, a call needs
+// nothing that it would not have held with the one-launch tile (the same bits): that one runs
+// where the call keeps no scratch (so that calls may run on several streams at once, and a captured
+// one owns all it writes) or there is no memory for the work field.
 int call_tile(sp_prop* p, int nslices, int f64, bool scratch, bool aligned, FusedTile* t)
 {
     *t = pick_tile(p, nslices, f64);
-    const bool builtin = p->tile.tx == 0 && !p->tuned.count({nslices, f64 ? 1 : 0});
-    if (builtin && !aligned && p->tile.kchunk < 0)
+    const bool set = p->tile.tx > 0;
+    if (!set && !aligned && p->tile.kchunk < 0 && !p->tuned.count({nslices, f64 ? 1 : 0}))
         *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, false, false);
     if (t->variant != SP_KERNEL_SPLIT) return SP_OK;
-    if (scratch || !builtin) {
+    if (scratch || set) {
         const int r = ensure_split(p, *t, nslices);
-        if (r == SP_OK || !builtin) return r;
+        if (r == SP_OK || set) return r;
         (void)hipGetLastError();  // the allocation's
     }
     *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, true);
@@ -323,7 +323,7 @@ int rk4_fused_run(sp_prop* p, int idt, View vin, int odt, View vout, bool aliase
     FusedTile tile;
     // later steps run between the output and the scratch, whose rows are ni long
     const bool aligned = pairs_aligned(vout, odt) && (steps > 1 || pairs_aligned(vin, idt));
-    SP_TRY(call_tile(p, 1, idt == SP_F64 && odt == SP_F64, true, aligned, &tile));
+    SP_TRY(call_tile(p, 1, idt == SP_F64 && odt == SP_F64, steps > 1 || aliased, aligned, &tile));
     const View A = cview(p->scratch[0].p, p->ni, p->nj), B = cview(p->scratch[1].p, p->ni, p->nj);
     View src = vin;
     int sdtype = idt;
