@@ -146,18 +146,34 @@ FusedStep fused_step(const sp_prop* p, int nslices, double dt, const void* coef_
     return st;
 }
 
-// The work field a split tile needs for `nslices` slices; nothing for the other variants.
-// Called where a tile is picked, before any launch is captured.
-int ensure_split(sp_prop* p, const FusedTile& t, int nslices)
+bool capturing(hipStream_t s)
 {
-    if (t.variant != SP_KERNEL_SPLIT) return SP_OK;
-    return p->split.ensure(split_work_bytes(p->ni, p->nj, p->nk, nslices));
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
+// The work field that split steps of `nslices` slices need.  A captured call's stays where it is:
+// a larger field is a new one beside it.
+int ensure_split(sp_prop* p, int nslices, bool captured)
+{
+    const size_t bytes = split_work_bytes(p->ni, p->nj, p->nk, nslices);
+    if (bytes > p->split.cap && p->split_captured) {
+        p->split_kept.push_back(p->split.p);
+        p->split = Buf{};
+        p->split_captured = false;
+    }
+    SP_TRY(p->split.ensure(bytes));
+    p->split_captured |= captured;
+    return SP_OK;
 }
 
 // The tile of a step's call, its work field there.  Unless the caller set the tile, a call needs
 // nothing that it would not have held with the one-launch tile (the same bits): that one runs
 // where the call keeps no scratch (so that calls may run on several streams at once, and a captured
-// one owns all it writes) or there is no memory for the work field.
+// one owns all it writes), where there is no memory for the work field, and where it would have to
+// be allocated under capture.
 int call_tile(sp_prop* p, int nslices, int f64, bool scratch, bool aligned, FusedTile* t)
 {
     *t = pick_tile(p, nslices, f64);
@@ -165,8 +181,10 @@ int call_tile(sp_prop* p, int nslices, int f64, bool scratch, bool aligned, Fuse
     if (!set && !aligned && p->tile.kchunk < 0 && !p->tuned.count({nslices, f64 ? 1 : 0}))
         *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, false, false);
     if (t->variant != SP_KERNEL_SPLIT) return SP_OK;
-    if (scratch || set) {
-        const int r = ensure_split(p, *t, nslices);
+    const bool cap = capturing(p->ctx->stream);
+    const bool there = split_work_bytes(p->ni, p->nj, p->nk, nslices) <= p->split.cap;
+    if (set || (scratch && (there || !cap))) {
+        const int r = ensure_split(p, nslices, cap);
         if (r == SP_OK || set) return r;
         (void)hipGetLastError();  // the allocation's
     }
@@ -275,11 +293,18 @@ int tune_fused(sp_prop* p, int nslices, int idt, int odt, View in, View out, dou
     if (tune_memo_hit(p, nslices, idt, odt, best_us)) return SP_OK;
     std::vector<FusedTile> cand;
     fused_candidates(p->ni, p->nj, p->nk, nslices, f64, cand);
-    for (const FusedTile& t : cand) SP_TRY(ensure_split(p, t, nslices));
+    // a work field of its own: the propagator's stays as calls before and after know it
+    struct Work : Buf {
+        ~Work() { release(); }
+    } work;
+    for (const FusedTile& t : cand)
+        if (t.variant == SP_KERNEL_SPLIT) SP_TRY(work.ensure(split_work_bytes(p->ni, p->nj, p->nk, nslices)));
     hipEvent_t e0, e1;
     SP_HIP(hipEventCreate(&e0));
     SP_HIP(hipEventCreate(&e1));
-    const FusedStep st = fused_step(p, nslices, 1e-6, nullptr, p->nu0);
+    FusedStep st = fused_step(p, nslices, 1e-6, nullptr, p->nu0);
+    st.work = work.p;
+    st.work_bytes = work.cap;
     std::vector<std::pair<double, size_t>> times;
     int r = SP_OK;
     for (size_t i = 0; i < cand.size() && r == SP_OK; ++i) {
@@ -574,6 +599,7 @@ static void prop_release(sp_prop* p)
     (void)hipStreamSynchronize(p->ctx->stream);
     for (Buf* b : {&p->scratch[0], &p->scratch[1], &p->split, &p->qI, &p->k1, &p->k2, &p->k3, &p->k4, &p->nu_tab})
         b->release();
+    for (void* w : p->split_kept) (void)hipFree(w);
     sp_ctx* c = p->ctx;
     delete p;
     ctx_release(c);

@@ -95,3 +95,27 @@ def test_captured_single_step_after_larger_calls(sp, shape):
         g.replay()
         torch.cuda.synchronize()
         assert np.array_equal(b.get(), scalar_steps(sp, shape, seeded(shape, i), 1))
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 64), (63, 64, 64)], ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("warm", [False, True])
+def test_captured_steps_after_larger_calls(sp, shape, warm):
+    """Several steps captured once the scratch is there: without a work field (never used before)
+    and with one, which later calls, all within the scratch, and the autotuner outgrow."""
+    conv = convection(sp, shape)
+    batched(conv, 64, 2)  # too many bricks for the built-in choice: a scratch of 64 slices, no work field
+    a, b = conv.field(), conv.field()
+    a.set(seeded(shape, 0))
+    if warm:
+        conv.DoRK4(a, b, 0.0, 1e-4, 3)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        conv.DoRK4(a, b, 0.0, 1e-4, 3)
+    for i, later in enumerate((lambda: batched(conv, 5, 3), lambda: conv.autotune(7), lambda: batched(conv, 9, 2))):
+        later()
+        a.set(seeded(shape, i))
+        b.set(np.zeros(shape[::-1]))
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(b.get(), scalar_steps(sp, shape, seeded(shape, i), 3))
