@@ -1352,14 +1352,35 @@ int sp_parareal_create(sp_prop* p, const sp_parareal_cfg* cfg, sp_parareal** out
     pr->tileGS = pick_tile(p, pr->S, pr->gdt == SP_F64);
     pr->tileG1_64 = pick_tile(p, 1, 1);
     {
+        // The work field of the split tiles that this configuration launches.  The others, and all
+        // of them if there is no memory for it, are one-launch tiles (the same bits) unless set by
+        // the caller.
+        const bool set = p->tile.tx > 0, fused = p->path == SP_PATH_FUSED, rk4 = cfg->coarse_kind == SP_COARSE_RK4;
+        const bool init64 = cfg->initial_fp64 && pr->gdt != SP_F64;
+        struct Use {
+            FusedTile* tile;
+            int nslices;
+            bool launched;
+        };
+        std::vector<Use> uses{{&pr->tileF, pr->S, fused}, {&pr->tileG1_64, 1, fused && rk4 && init64}};
+        if (pr->gdt == SP_F64) {
+            uses.push_back({&pr->tileG1, 1, fused && rk4});
+            uses.push_back({&pr->tileGS, pr->S, fused && rk4 && !cfg->delta_correction && !pr->nu_const});
+        }
+        const auto one_launch = [&](const Use& u) {
+            if (u.tile->variant == SP_KERNEL_SPLIT) *u.tile = default_tile(p->ni, p->nj, p->nk, u.nslices, 1, true);
+        };
         size_t wb = 0;
-        if (pr->tileG1_64.variant == SP_KERNEL_SPLIT) wb = split_work_bytes(p->ni, p->nj, p->nk, 1);
-        if (pr->tileF.variant == SP_KERNEL_SPLIT) wb = std::max(wb, split_work_bytes(p->ni, p->nj, p->nk, pr->S));
-        if (pr->gdt == SP_F64 && pr->tileG1.variant == SP_KERNEL_SPLIT)
-            wb = std::max(wb, split_work_bytes(p->ni, p->nj, p->nk, 1));
-        if (pr->gdt == SP_F64 && pr->tileGS.variant == SP_KERNEL_SPLIT)
-            wb = std::max(wb, split_work_bytes(p->ni, p->nj, p->nk, pr->S));
-        const int r = wb ? pr->W.ensure(wb) : SP_OK;
+        for (const Use& u : uses) {
+            if (!u.launched && !set) one_launch(u);
+            if (u.tile->variant == SP_KERNEL_SPLIT) wb = std::max(wb, split_work_bytes(p->ni, p->nj, p->nk, u.nslices));
+        }
+        int r = wb ? pr->W.ensure(wb) : SP_OK;
+        if (r == SP_ERR_NOMEM && !set) {
+            (void)hipGetLastError();  // the allocation's
+            for (const Use& u : uses) one_launch(u);
+            r = SP_OK;
+        }
         if (r != SP_OK) {
             sp_parareal_destroy(pr);
             return r;
