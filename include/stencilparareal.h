@@ -119,7 +119,8 @@ int sp_prop_set_upwind(sp_prop* p, int upwind);
 int sp_prop_set_path(sp_prop* p, int path);
 /* Fused-kernel choice: variant SP_KERNEL_*, tile tx x ty columns, nthreads per block,
  * kchunk planes per block (0: whole k extent).  variant SP_KERNEL_AUTO restores the
- * built-in choice.  Compiled shapes: scalar {32x32x1024, 32x24x1024, 24x24x1024,
+ * built-in choice; with kchunk > 0 among the kernels that walk k, in chunks of that many
+ * planes.  Compiled shapes: scalar {32x32x1024, 32x24x1024, 24x24x1024,
  * 32x16x512, 16x16x256}, pair {32x32x512, 32x16x512, 16x16x256}, quad {32x32x512}
  * (its blocks run 768 threads; the built-in choice for FP64, but for fields of few bricks;
  * FP32 / BF16 storage takes the pair kernel in its place), split {32x32x512,

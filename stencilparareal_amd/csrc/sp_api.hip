@@ -123,7 +123,11 @@ FusedTile pick_tile(const sp_prop* p, int nslices, int f64)
         t.nt = p->tile.nt;
         t.variant = p->tile.variant;
     }
-    if (p->tile.kchunk >= 0) t.kchunk = p->tile.kchunk;
+    if (p->tile.kchunk >= 0) {
+        // a k chunk set alone is one of a kernel that walks k: bricks have none
+        if (p->tile.tx == 0 && fused_tile_brick(t)) t = default_tile(p->ni, p->nj, p->nk, nslices, f64, true);
+        t.kchunk = p->tile.kchunk;
+    }
     return t;
 }
 

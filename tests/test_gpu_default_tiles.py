@@ -92,3 +92,21 @@ def test_default_tile_odd_rows(sp, n, steps):
         torch.cuda.synchronize()
         out.append(b)
     assert torch.isfinite(out[1]).all() and torch.equal(*out)
+
+
+@pytest.mark.parametrize("shape", [(48, 48, 40), (47, 48, 40), (192, 192, 192)], ids=lambda s: "%dx%dx%d" % s)
+def test_k_chunk_set_alone(sp, shape):
+    """A k chunk without a tile is the chunk of the kernel that runs, whatever the size's own choice."""
+    ni, nj, nk = shape
+    q0 = np.random.default_rng(ni).standard_normal((nk, nj, ni))
+    out = []
+    for kwargs in (dict(kchunk=12), dict(tx=32, ty=16, nthreads=512, variant="scalar")):
+        conv = sp.Convection(ni, nj, nk, 1. / 64, 0.02, 0.0, 1.0, -0.5, 0.25)
+        conv.set_tile(**kwargs)
+        tile = conv.get_tile(1)
+        assert tile["variant"] != "split" and tile["kchunk"] == kwargs.get("kchunk", 0)
+        a, b = conv.field(), conv.field()
+        a.set(q0)
+        conv.DoRK4(a, b, 0.0, 1e-4, 3)
+        out.append(b.get())
+    assert np.isfinite(out[1]).all() and np.array_equal(*out)
