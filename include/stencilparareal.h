@@ -129,7 +129,8 @@ int sp_prop_set_path(sp_prop* p, int path);
  * of the batch) when the tile is chosen; its results equal the other FP64 variants' bit
  * for bit.  Its shape 16x16x384 computes bricks of 16x16x8 points (whatever kchunk says, in
  * blocks of 640 threads), on any sizes and strides; the other shapes need an even ni.  Grouped
- * batches (sp_batch_*) and sp_do_rk4_noalloc run the built-in one-launch choice in its place, as
+ * batches (sp_batch_*) and sp_do_rk4_noalloc run a one-launch tile in its place (the fastest that
+ * sp_prop_autotune timed, else the built-in choice), as
  * do calls without a tile set where there is no memory for the work field, and those of a single
  * step with in != out, which use nothing but in and out: calls of that kind may run on several
  * streams at once, and a captured one stays valid whatever the propagator runs later. */
@@ -147,8 +148,9 @@ int sp_prop_get_tile(const sp_prop* p, int nslices, int f64, int* variant, int* 
  * times every compiled fused-kernel tile shape and k chunk for `nslices` slices of this
  * propagator's size with the given storage types, and keeps the fastest for later
  * sp_do_rk4* calls with that slice count and compute type (FP64 when both types are
- * SP_F64, else FP32), unless a tile is set with sp_prop_set_tile.  Each candidate runs for
- * about 2 ms of timed launches and the two fastest are timed again.  Results are kept for
+ * SP_F64, else FP32), unless a tile is set with sp_prop_set_tile; where a split tile is the
+ * fastest, the fastest one-launch tile is kept beside it.  Each candidate runs for
+ * about 2 ms of timed launches and the two fastest of each kind are timed again.  Results are kept for
  * the process per (device, sizes, slice count, storage types), so later propagators and
  * Parareal objects of the same sizes reuse them without timing; with the environment
  * variable SP_AUTOTUNE_CACHE set to a file path they are also read from and appended to

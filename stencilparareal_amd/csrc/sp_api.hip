@@ -116,7 +116,7 @@ FusedTile pick_tile(const sp_prop* p, int nslices, int f64)
 {
     FusedTile t = default_tile(p->ni, p->nj, p->nk, nslices, f64);
     const auto hit = p->tuned.find({nslices, f64 ? 1 : 0});
-    if (p->tile.tx == 0 && hit != p->tuned.end()) return hit->second;
+    if (p->tile.tx == 0 && hit != p->tuned.end()) return hit->second.best;
     if (p->tile.tx > 0) {
         t.tx = p->tile.tx;
         t.ty = p->tile.ty;
@@ -130,6 +130,17 @@ FusedTile pick_tile(const sp_prop* p, int nslices, int f64)
     }
     return t;
 }
+
+}  // namespace
+
+FusedTile one_launch_tile(const sp_prop* p, int nslices, int f64)
+{
+    const auto hit = p->tuned.find({nslices, f64 ? 1 : 0});
+    if (p->tile.tx == 0 && hit != p->tuned.end() && hit->second.one_launch.tx > 0) return hit->second.one_launch;
+    return default_tile(p->ni, p->nj, p->nk, nslices, f64, true);
+}
+
+namespace {
 
 FusedStep fused_step(const sp_prop* p, int nslices, double dt, const void* coef_dev, double nu)
 {
@@ -192,7 +203,7 @@ int call_tile(sp_prop* p, int nslices, int f64, bool scratch, bool aligned, Fuse
         if (r == SP_OK || set) return r;
         (void)hipGetLastError();  // the allocation's
     }
-    *t = default_tile(p->ni, p->nj, p->nk, nslices, f64, true);
+    *t = one_launch_tile(p, nslices, f64);
     return SP_OK;
 }
 
@@ -216,7 +227,20 @@ struct TuneKey {
     }
 };
 std::mutex g_tune_mu;
-std::map<TuneKey, std::pair<FusedTile, double>> g_tune_memo;
+// The fastest tile of those in one launch and of the split ones, with their times (tx == 0: none).
+struct TuneResult {
+    FusedTile one_launch{}, split{};
+    double one_us = 0., split_us = 0.;
+    void add(const FusedTile& t, double us)
+    {
+        (t.variant == SP_KERNEL_SPLIT ? split : one_launch) = t;
+        (t.variant == SP_KERNEL_SPLIT ? split_us : one_us) = us;
+    }
+    bool split_best() const { return split.tx > 0 && (one_launch.tx == 0 || split_us < one_us); }
+    Tuned tuned() const { return {split_best() ? split : one_launch, one_launch}; }
+    double us() const { return split_best() ? split_us : one_us; }
+};
+std::map<TuneKey, TuneResult> g_tune_memo;
 bool g_tune_file_read = false;
 
 void tune_cache_read_locked()
@@ -232,13 +256,13 @@ void tune_cache_read_locked()
     double us;
     while (std::fscanf(f, "%d %d %d %d %d %d %d %d %d %d %d %d %lf", &k.dev, &k.ni, &k.nj, &k.nk, &k.nslices, &k.idt,
                        &k.odt, &t.variant, &t.tx, &t.ty, &t.nt, &t.kchunk, &us) == 13)
-        if (fused_tile_supported(t, 1)) g_tune_memo[k] = {t, us};
+        if (fused_tile_supported(t, 1)) g_tune_memo[k].add(t, us);
     std::fclose(f);
 }
 
 void tune_cache_write_locked(const TuneKey& k, const FusedTile& t, double us)
 {
-    g_tune_memo[k] = {t, us};
+    g_tune_memo[k].add(t, us);
     const char* path = std::getenv("SP_AUTOTUNE_CACHE");
     if (!path || !*path) return;
     if (FILE* f = std::fopen(path, "a")) {
@@ -281,8 +305,8 @@ bool tune_memo_hit(sp_prop* p, int nslices, int idt, int odt, double* best_us)
     tune_cache_read_locked();
     const auto hit = g_tune_memo.find(key);
     if (hit == g_tune_memo.end()) return false;
-    p->tuned[{nslices, idt == SP_F64 && odt == SP_F64 ? 1 : 0}] = hit->second.first;
-    if (best_us) *best_us = hit->second.second;
+    p->tuned[{nslices, idt == SP_F64 && odt == SP_F64 ? 1 : 0}] = hit->second.tuned();
+    if (best_us) *best_us = hit->second.us();
     return true;
 }
 
@@ -316,27 +340,32 @@ int tune_fused(sp_prop* p, int nslices, int idt, int odt, View in, View out, dou
         r = time_tile(s, st, cand[i], idt, in, odt, out, e0, e1, &us);
         times.push_back({us, i});
     }
-    // the two fastest once more, so a single noisy timing does not decide
-    if (r == SP_OK && times.size() > 1) {
-        std::sort(times.begin(), times.end());
-        for (int j = 0; j < 2 && r == SP_OK; ++j) {
+    // the two fastest of each kind once more, so a single noisy timing does not decide
+    std::sort(times.begin(), times.end());
+    TuneResult best;
+    for (const bool split : {false, true}) {
+        std::vector<std::pair<double, size_t>> kind;
+        for (const auto& x : times)
+            if ((cand[x.second].variant == SP_KERNEL_SPLIT) == split && kind.size() < 2) kind.push_back(x);
+        for (size_t j = 0; j < kind.size() && kind.size() > 1 && r == SP_OK; ++j) {
             double us = 0.;
-            r = time_tile(s, st, cand[times[j].second], idt, in, odt, out, e0, e1, &us);
-            times[j].first = std::min(times[j].first, us);
+            r = time_tile(s, st, cand[kind[j].second], idt, in, odt, out, e0, e1, &us);
+            kind[j].first = std::min(kind[j].first, us);
         }
-        std::sort(times.begin(), times.begin() + 2);
+        std::sort(kind.begin(), kind.end());
+        if (!kind.empty()) best.add(cand[kind.front().second], kind.front().first);
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     SP_TRY(r);
-    const FusedTile best_t = cand[times.front().second];
-    const double best = times.front().first;
-    p->tuned[{nslices, f64}] = best_t;
+    p->tuned[{nslices, f64}] = best.tuned();
     {
+        // a split tile is kept only where it is the fastest, its line the last one
         std::lock_guard<std::mutex> lock(g_tune_mu);
-        tune_cache_write_locked(key, best_t, best);
+        tune_cache_write_locked(key, best.one_launch, best.one_us);
+        if (best.split_best()) tune_cache_write_locked(key, best.split, best.split_us);
     }
-    if (best_us) *best_us = best;
+    if (best_us) *best_us = best.us();
     return SP_OK;
 }
 
@@ -755,9 +784,9 @@ int sp_do_rk4_noalloc(sp_prop* p, const sp_layout* lin, const void* in, const sp
     FusedTile tile = pick_tile(p, 1, 1);
     if (p->tile.tx == 0 && p->tile.kchunk < 0 && !p->tuned.count({1, 1}) && !pairs_aligned(vout, SP_F64))
         tile = default_tile(p->ni, p->nj, p->nk, 1, 1, true);
-    // the split steps need a second intermediate field: the built-in one-launch tile instead
+    // the split steps need a second intermediate field: the one-launch tile instead
     // (the same result bit for bit)
-    if (tile.variant == SP_KERNEL_SPLIT) tile = default_tile(p->ni, p->nj, p->nk, 1, 1, true);
+    if (tile.variant == SP_KERNEL_SPLIT) tile = one_launch_tile(p, 1, 1);
     // out and A alternate so the last step lands in out; in place (in == out), the first
     // step must not write in, so an odd count ends in A and is copied to out
     View src = vin;
@@ -1372,7 +1401,7 @@ int sp_parareal_create(sp_prop* p, const sp_parareal_cfg* cfg, sp_parareal** out
             uses.push_back({&pr->tileGS, pr->S, fused && rk4 && !cfg->delta_correction && !pr->nu_const});
         }
         const auto one_launch = [&](const Use& u) {
-            if (u.tile->variant == SP_KERNEL_SPLIT) *u.tile = default_tile(p->ni, p->nj, p->nk, u.nslices, 1, true);
+            if (u.tile->variant == SP_KERNEL_SPLIT) *u.tile = one_launch_tile(p, u.nslices, 1);
         };
         size_t wb = 0;
         for (const Use& u : uses) {

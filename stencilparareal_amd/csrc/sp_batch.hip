@@ -428,11 +428,11 @@ int sp_batch_create(sp_ctx* ctx, int nprob, const sp_problem* probs, const sp_ba
             int v = 0;
             chk(sp_prop_get_tile(q.prop, nslices, f64, &v, &t.tx, &t.ty, &t.nt, &t.kchunk));
             t.variant = v;
-            // Grouped launches have no split form: the built-in one-launch tile.  Nor the coarse
+            // Grouped launches have no split form: the one-launch tile.  Nor the coarse
             // chain the tile that is fastest by itself: problems of one tile shape share a launch,
             // which fills the chip (six problems of 64^3 to 160^3: 71 ms a pass against 78 ms).
             if (t.variant == SP_KERNEL_SPLIT || (!f64 && !cfg->autotune && nprob > 1))
-                t = default_tile(q.d.n, q.d.n, q.d.n, nslices, f64, true);
+                t = one_launch_tile(q.prop, nslices, f64);
             tuned[key] = t;
         };
         if (shared_fine)

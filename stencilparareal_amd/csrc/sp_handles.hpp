@@ -43,6 +43,12 @@ struct Buf {
     }
 };
 
+// The autotuner's choice: the fastest tile, and the fastest of those that step in one launch (the
+// same one unless a split tile is fastest; tx == 0: not measured).
+struct Tuned {
+    sp::FusedTile best, one_launch;
+};
+
 struct sp_prop {
     int refs = 1;
     sp_ctx* ctx = nullptr;
@@ -58,5 +64,8 @@ struct sp_prop {
     Buf qI, k1, k2, k3, k4;         // staged path temporaries (f64, compact)
     Buf nu_tab;                     // per-step nu table
     std::vector<double> nu_host;
-    std::map<std::pair<int, int>, sp::FusedTile> tuned;  // (slices, FP64 compute) -> autotuned tile
+    std::map<std::pair<int, int>, Tuned> tuned;  // (slices, FP64 compute) -> autotuned tiles
 };
+
+// The propagator's choice among the tiles that step in one launch without a work field.
+sp::FusedTile one_launch_tile(const sp_prop* p, int nslices, int f64);
