@@ -129,9 +129,9 @@ int sp_prop_set_path(sp_prop* p, int path);
  * of the batch) when the tile is chosen; its results equal the other FP64 variants' bit
  * for bit.  Its shape 16x16x384 computes bricks of 16x16x8 points (whatever kchunk says, in
  * blocks of 640 threads), on any sizes and strides; the other shapes need an even ni.  Grouped
- * batches (sp_batch_*) and sp_do_rk4_noalloc run a one-launch tile in its place (the fastest that
- * sp_prop_autotune timed, else the built-in choice), as
- * do calls without a tile set where there is no memory for the work field, and those of a single
+ * batches (sp_batch_*) run the built-in one-launch choice in its place; sp_do_rk4_noalloc runs a
+ * one-launch tile (the fastest that sp_prop_autotune timed, else the built-in choice), as do
+ * calls without a tile set where there is no memory for the work field, and those of a single
  * step with in != out, which use nothing but in and out: calls of that kind may run on several
  * streams at once, and a captured one stays valid whatever the propagator runs later. */
 int sp_prop_set_tile(sp_prop* p, int variant, int tx, int ty, int nthreads, int kchunk);

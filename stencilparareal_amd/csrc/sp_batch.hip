@@ -428,11 +428,16 @@ int sp_batch_create(sp_ctx* ctx, int nprob, const sp_problem* probs, const sp_ba
             int v = 0;
             chk(sp_prop_get_tile(q.prop, nslices, f64, &v, &t.tx, &t.ty, &t.nt, &t.kchunk));
             t.variant = v;
-            // Grouped launches have no split form: the one-launch tile.  Nor the coarse
-            // chain the tile that is fastest by itself: problems of one tile shape share a launch,
-            // which fills the chip (six problems of 64^3 to 160^3: 71 ms a pass against 78 ms).
+            // Grouped launches have no split form: the built-in one-launch tile, also where a split tile
+            // was tuned.  The fastest one-launch tiles timed problem by problem differ in shape, so
+            // that problems no longer share a launch (64^3 x 8 and 160^3 x 8, FP64: fine sweeps 6.5 ms
+            // against 4.0; 64^3 to 160^3, six problems: 23.1 against 20.7).  Nor has the coarse chain in
+            // FP32 / BF16 the tile that is fastest by itself: problems of one tile shape share a launch,
+            // which fills the chip (six problems of 64^3 to 160^3: 71 ms a pass against 78 ms).  In
+            // FP64 their own tiles are faster (the two problems' chains 3.1 ms against 3.6, four of
+            // 160^3 6.8 against 9.6, 112^3 to 256^3 9.3 against 18.6).
             if (t.variant == SP_KERNEL_SPLIT || (!f64 && !cfg->autotune && nprob > 1))
-                t = one_launch_tile(q.prop, nslices, f64);
+                t = default_tile(q.d.n, q.d.n, q.d.n, nslices, f64, true);
             tuned[key] = t;
         };
         if (shared_fine)

