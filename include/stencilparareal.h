@@ -57,7 +57,7 @@ extern "C" {
 #define SP_KERNEL_SCALAR 0 /* one column per lane, any sizes and storage types */
 #define SP_KERNEL_PAIR 1   /* two x-adjacent columns per lane: FP64 (16-byte accesses) or FP32 arithmetic over FP32 / BF16 storage */
 #define SP_KERNEL_QUAD 2   /* FP64, 2x2 columns per lane (32x32 tiles) */
-#define SP_KERNEL_SPLIT 3  /* FP64, two launches of a two-stage x-pair kernel through a work field */
+#define SP_KERNEL_SPLIT 3  /* FP64, two launches of a two-stage kernel through a work field: x-pair tiles or bricks */
 
 /*
  * Field layout.  Element (i,j,k) of the interior, 0 <= i < ni etc., lives at
@@ -135,13 +135,16 @@ int sp_prop_set_path(sp_prop* p, int path);
  * step with in != out, which use nothing but in and out: calls of that kind may run on several
  * streams at once, and a captured one stays valid whatever the propagator runs later. */
 int sp_prop_set_tile(sp_prop* p, int variant, int tx, int ty, int nthreads, int kchunk);
-/* The fused-kernel tile sp_do_rk4 (nslices = 1) or sp_do_rk4_batched (nslices > 1) will
- * use for FP64 compute (f64 = 1) or reduced-precision storage (f64 = 0): the one set with
- * sp_prop_set_tile, else the built-in choice for this size.  Output pointers may be NULL.
- * Fields the pair, quad and split kernels cannot take (odd ni, odd strides, origins not
- * aligned to two elements; quad and split: storage other than FP64) run the scalar
- * 32x16x512 kernel instead; the report covers odd ni and f64 = 0 (no counterpart in the
- * reference). */
+/* The fused-kernel tile that sp_do_rk4 (nslices = 1) or sp_do_rk4_batched (nslices > 1) uses
+ * for FP64 compute (f64 = 1) or reduced-precision storage (f64 = 0) in a call of several steps
+ * on fields with even strides and origins aligned to two elements: the one set with
+ * sp_prop_set_tile, else the autotuned one, else the built-in choice for this size.  Output
+ * pointers may be NULL.  Fields the pair, quad and split kernels cannot take (odd ni, odd
+ * strides, other origins; quad and split: storage other than FP64) run the scalar 32x16x512
+ * kernel instead, except with the split variant's bricks, which take any FP64 field; the report
+ * covers odd ni and f64 = 0.  Not in the report: without a tile set, FP64 fields of odd strides
+ * or other origins take bricks while those are few, and the calls named at sp_prop_set_tile a
+ * one-launch tile (no counterpart in the reference). */
 int sp_prop_get_tile(const sp_prop* p, int nslices, int f64, int* variant, int* tx, int* ty, int* nthreads,
                      int* kchunk);
 /* Autotuner (no counterpart in the reference, whose CUDA block size is fixed at 32x4):

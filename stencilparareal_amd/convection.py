@@ -39,7 +39,7 @@ class Convection:
     def set_tile(self, tx=0, ty=0, nthreads=0, kchunk=0, variant=None):
         """Fused-kernel tile.  variant: "scalar", "pair", "quad" (FP64 32x32x512 only), "split"
         (FP64, two launches of a two-stage kernel) or None (built-in choice when tx == 0, else
-        scalar)."""
+        scalar).  kchunk alone: the k chunk of the built-in choice."""
         if tx == 0 and variant is None:
             v = L.SP_KERNEL_AUTO
         else:
@@ -48,7 +48,8 @@ class Convection:
         L.call("sp_prop_set_tile", self.h, v, tx, ty, nthreads, kchunk)
 
     def get_tile(self, nslices: int = 1, f64: bool = True) -> dict:
-        """The fused-kernel tile a call with `nslices` slices launches."""
+        """The fused-kernel tile of a call of several steps with `nslices` slices
+        (sp_prop_get_tile)."""
         v = [C.c_int() for _ in range(5)]
         L.call("sp_prop_get_tile", self.h, nslices, 1 if f64 else 0, *[C.byref(x) for x in v])
         var, tx, ty, nt, kc = (x.value for x in v)

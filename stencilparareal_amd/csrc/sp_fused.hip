@@ -2177,7 +2177,7 @@ FusedTile default_tile(int ni, int nj, int nk, int nslices, int compute_f64, boo
     // FP32, us per plane (BF16 5-20 % more): 32x32 1.46 per round, 32x16 1.05 alone and 0.78 per
     // round of two and more, 16x16 0.88 and 0.60.  1 x 64^3 16x16 in 8-plane chunks 23.6 us (34.5
     // for 32x16 in 16), 1 x 256^3 32x32 in 64 122 (154 for 32x16 in 128), 1 x 384^3 32x32 in 77-80
-    // 435 (479 in 64; BF16 526 against 598, its best, 32x16 in 64, 499).
+    // 420 (479 in 64; BF16 526 against 598, its best, 32x16 in 64, 499).
     if (!compute_f64 && !one_launch && pairs) {
         static constexpr struct {
             int tx, ty, nt;
