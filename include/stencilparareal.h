@@ -148,7 +148,7 @@ int sp_prop_set_tile(sp_prop* p, int variant, int tx, int ty, int nthreads, int 
 int sp_prop_get_tile(const sp_prop* p, int nslices, int f64, int* variant, int* tx, int* ty, int* nthreads,
                      int* kchunk);
 /* Autotuner (no counterpart in the reference, whose CUDA block size is fixed at 32x4):
- * times every compiled fused-kernel tile shape and k chunk for `nslices` slices of this
+ * times every compiled fused-kernel tile shape in a set of k chunks for `nslices` slices of this
  * propagator's size with the given storage types, and keeps the fastest for later
  * sp_do_rk4* calls with that slice count and compute type (FP64 when both types are
  * SP_F64, else FP32), unless a tile is set with sp_prop_set_tile; where a split tile is the
