@@ -42,3 +42,26 @@ def test_euler_steps_brick_edges(shape, steps):
 @pytest.mark.parametrize("kind,in_place", [("stella", False), ("compact", True)])
 def test_euler_steps_padded_and_in_place(steps, kind, in_place):
     check((40, 20, 17), steps, 1. / 32, True, kind=kind, in_place=in_place)
+
+
+@pytest.mark.parametrize("steps", [2, 4, 6, 10])
+@pytest.mark.parametrize("shift", [2, 33, 32 * 32 * 9])
+def test_euler_steps_overlapping_storage(steps, shift):
+    """An output that overlaps the input `shift` points on: an even number of steps reads the input
+    only while it writes to the scratch."""
+    import ctypes as C
+    import stencilparareal_amd as sp
+    from stencilparareal_amd import _lib as L
+    n, c = 32, (1.0, -0.5, 0.25)
+    conv = sp.Convection(n, n, n, 1. / n, 0.01, 30.0, *c)
+    lay = L.Layout()
+    L.call("sp_layout_compact", n, n, n, L.SP_F64, C.byref(lay))
+    q0 = np.random.default_rng(shift + steps).standard_normal((n, n, n))
+    buf = torch.zeros(n**3 + shift, dtype=torch.float64, device="cuda")
+    buf[:n**3] = torch.from_numpy(q0.ravel())
+    conv.ctx.sync_stream()
+    L.call("sp_do_euler", conv.h, C.byref(lay), C.c_void_p(buf.data_ptr()), C.byref(lay),
+           C.c_void_p(buf.data_ptr() + 8 * shift), 0.2, 1e-4, steps)
+    torch.cuda.synchronize()
+    want = O.OConvection(n, n, n, 1. / n, 0.01, 30.0, *c).euler(q0, 0.2, 1e-4, steps)
+    assert np.array_equal(buf[shift:].cpu().numpy().reshape(n, n, n), want)
